@@ -1,109 +1,107 @@
-// The dW split-K reduce (experts.hip's dw_reduce kernels; also run inside combine_dx's
+// The dW split-K reduce (experts.hip's dw_reduce_kernel; also run inside combine_dx's
 // launch, router_grad.hip): the fp32 partials of the multi-chunk groups summed in chunk
-// order into dW.  The workgroup's column of the pass (bx of nbx) is an argument, so the
-// body runs in any launch whose workgroups have NT threads.
+// order into dW.  The workgroup's index is an argument, so the body runs in any launch whose
+// workgroups have NT threads.
 #pragma once
 
 #include "experts_common.h"
 
 namespace nsmoe {
 
-// Workgroup bx of nbx sums group g's partials: each thread 4 consecutive elements (one
-// 16-byte vector per chunk, every chunk's load in flight at once), so the pass streams
-// the partials at full width; the order of the additions is the chunk order for every
-// element, whatever the launch shape.
-template <int DT, int MODE>
-__device__ __forceinline__ void dw_reduce_group(const ExpParams& p, int g, int bx, int nbx) {
-  using T = typename Elem<DT>::T;
-  const int nch = dw_chunks(rows_of(p, g));
-  if (nch <= 1) return;
-  // First partial of group g: the chunk counts of the multi-chunk groups before it,
-  // counted by all threads at once (integer sum: the order does not matter).  A caller
-  // may run several groups in turn (dw_reduce_pair_row): the barrier before the reset
-  // keeps thread 0 from clearing s_base while a slower wave still reads the previous
-  // group's value.
-  __shared__ int s_base;
-  __syncthreads();
-  if (threadIdx.x == 0) s_base = 0;
-  __syncthreads();
-  int part = 0;
-  for (int q = threadIdx.x; q < g; q += NT) {
-    const int c = dw_chunks(rows_of(p, q));
-    if (c > 1) part += c;
-  }
-  if (part) atomicAdd(&s_base, part);
-  __syncthreads();
-  const int d = p.d, H = p.H;
-  const int64_t mn = MODE == 0 ? (int64_t)d * 2 * H : (int64_t)H * d;
-  T* dst = g < p.E ? (T*)p.dw_a + (int64_t)g * mn : (T*)p.dw_sh + (int64_t)(g - p.E) * mn;
-  const float* src = p.partial + (int64_t)s_base * mn;
-  const int64_t n4 = (mn % 4 == 0) ? mn / 4 : 0;  // 16-byte vectors (every partial is 16-B aligned)
-  for (int64_t i = (int64_t)bx * NT + threadIdx.x; i < n4; i += (int64_t)nbx * NT) {
-    // Up to DEPTH chunks' loads in flight at once, added in chunk order.
+struct DwReduceArgs {
+  ExpParams p_in, p_out;  // dW_in and dW_out: pointers and partials
+  int wgs;                // workgroups (0: no reduce to run)
+};
+
+// Blocks of NT threads x 4 elements in one group's dW.
+__host__ __device__ __forceinline__ int dw_reduce_blocks(int64_t mn) {
+  return (int)((mn + 4 * NT - 1) / (4 * NT));
+}
+
+// Block b of the `nch` partials at `src` (mn elements each) into dst: each thread 4
+// consecutive elements, up to DEPTH chunks' 16-byte loads in flight at once; the additions
+// are in chunk order for every element, whatever the launch shape.
+template <int DT>
+__device__ __forceinline__ void dw_reduce_block(const float* src, int64_t mn, int nch, int b,
+                                                typename Elem<DT>::T* dst) {
+  const int64_t i = ((int64_t)b * NT + threadIdx.x) * 4;
+  if (i >= mn) return;
+  if (mn % 4 == 0) {  // every partial is 16-byte aligned
     constexpr int DEPTH = 16;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < nch; c0 += DEPTH) {
       f32x4 a[DEPTH];
 #pragma unroll
       for (int u = 0; u < DEPTH; ++u)
-        if (c0 + u < nch) a[u] = ((const f32x4*)(src + (int64_t)(c0 + u) * mn))[i];
+        if (c0 + u < nch) a[u] = *(const f32x4*)(src + (int64_t)(c0 + u) * mn + i);
 #pragma unroll
       for (int u = 0; u < DEPTH; ++u)
         if (c0 + u < nch) acc += a[u];
     }
-    if (DT != DT_F32 && ((uintptr_t)dst & 7) == 0) {  // one 8-byte store (mn % 4 == 0)
-      *(uint2*)(dst + i * 4) = make_uint2(pack2<DT>(acc[0], acc[1]), pack2<DT>(acc[2], acc[3]));
+    if (DT != DT_F32 && ((uintptr_t)dst & 7) == 0) {  // one 8-byte store
+      *(uint2*)(dst + i) = make_uint2(pack2<DT>(acc[0], acc[1]), pack2<DT>(acc[2], acc[3]));
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dst[i * 4 + e] = Elem<DT>::from_f(acc[e]);
+      for (int e = 0; e < 4; ++e) dst[i + e] = Elem<DT>::from_f(acc[e]);
     }
-  }
-  for (int64_t i = n4 * 4 + (int64_t)bx * NT + threadIdx.x; i < mn; i += (int64_t)nbx * NT) {
-    float acc = 0.0f;
-    for (int c = 0; c < nch; ++c) acc += src[(int64_t)c * mn + i];
-    dst[i] = Elem<DT>::from_f(acc);
+  } else {
+    for (int e = 0; e < 4 && i + e < mn; ++e) {
+      float acc = 0.0f;
+      for (int c = 0; c < nch; ++c) acc += src[(int64_t)c * mn + i + e];
+      dst[i + e] = Elem<DT>::from_f(acc);
+    }
   }
 }
 
-// Both modes over the groups that can have several chunks: row y in [0, 2 NY),
-// NY = S + routed_rows: mode = y / NY, row j = y % NY.  Rows j < S take shared group
-// E + j.  With routed_rows = E, row S + r takes routed group r; with routed_rows = 1 the
-// one row S finds the routed groups of several chunks (usually none or a few: routed
-// groups average fewer rows than a chunk) and takes them in turn.  A pass over all
-// 2 (E + S) groups spends most of its time on workgroups that only find one chunk.
-struct DwReduceArgs {
-  ExpParams p_in, p_out;  // dW_in and dW_out: pointers and partials
-  int routed_rows;
-  int nbx;                // workgroups per row (0: no reduce to run)
-  int rows;               // 2 (S + routed_rows)
-};
-
+// Workgroup wg of r.wgs.  The multi-chunk groups and their first partials are listed in LDS
+// (up to NT groups a round, shared groups first, as the partials lie), then the (group, mode,
+// block) items of the list are dealt over the workgroups: no barrier between items, so the
+// loads of one overlap the stores of the last.
 template <int DT>
-__device__ __forceinline__ void dw_reduce_pair_row(const DwReduceArgs& r, int bx, int y) {
-  const ExpParams& p_in = r.p_in;
-  const int E = p_in.E, S = p_in.S, ny = S + r.routed_rows;
-  const int mode = y >= ny ? 1 : 0, j = y - mode * ny;
-  auto run = [&](int g) {
-    if (mode == 0) dw_reduce_group<DT, 0>(r.p_in, g, bx, r.nbx);
-    else dw_reduce_group<DT, 1>(r.p_out, g, bx, r.nbx);
-  };
-  if (j < S) {
-    run(E + j);
-  } else if (r.routed_rows == E) {
-    run(j - S);
-  } else {
-    __shared__ int s_list[NT];
-    __shared__ int s_n;
-    for (int g0 = 0; g0 < E; g0 += NT) {
-      if (threadIdx.x == 0) s_n = 0;
-      __syncthreads();
-      const int g = g0 + (int)threadIdx.x;
-      if (g < E && dw_chunks(rows_of(p_in, g)) > 1) s_list[atomicAdd(&s_n, 1)] = g;
-      __syncthreads();
-      const int n = s_n;
-      for (int i = 0; i < n; ++i) run(s_list[i]);
-      __syncthreads();  // the list is read before the next round rewrites it
+__device__ __forceinline__ void dw_reduce_wg(const DwReduceArgs& r, int wg) {
+  using T = typename Elem<DT>::T;
+  __shared__ int s_g[NT], s_base[NT], s_sum[NT / 64], s_cnt[NT / 64];
+  const ExpParams& p = r.p_in;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t mn_in = (int64_t)p.d * 2 * p.H, mn_out = (int64_t)p.H * p.d;
+  const int b_in = dw_reduce_blocks(mn_in), nb = b_in + dw_reduce_blocks(mn_out);
+  int base = 0;
+  for (int v0 = 0; v0 < p.E + p.S; v0 += NT) {
+    const int v = v0 + tid;
+    const int g = v < p.S ? p.E + v : v - p.S;
+    int c = v < p.E + p.S ? dw_chunks(rows_of(p, g), p.dw_rc) : 0;
+    if (c <= 1) c = 0;
+    const int incl = wave_scan_incl(c);
+    const unsigned long long hit = __ballot(c > 0);
+    if (lane == 63) {
+      s_sum[wave] = incl;
+      s_cnt[wave] = __popcll(hit);
     }
+    __syncthreads();
+    int at = __popcll(hit & ((1ull << lane) - 1)), n = 0, first = base + incl - c;
+    for (int w = 0; w < NT / 64; ++w) {
+      if (w < wave) {
+        at += s_cnt[w];
+        first += s_sum[w];
+      }
+      n += s_cnt[w];
+      base += s_sum[w];
+    }
+    if (c) {
+      s_g[at] = g;
+      s_base[at] = first;
+    }
+    __syncthreads();
+    for (int64_t it = wg; it < (int64_t)n * nb; it += r.wgs) {
+      const int li = (int)(it / nb), b = (int)(it % nb);
+      const int gg = s_g[li], nch = dw_chunks(rows_of(p, gg), p.dw_rc);
+      const bool in = b < b_in;
+      const ExpParams& q = in ? r.p_in : r.p_out;
+      const int64_t mn = in ? mn_in : mn_out;
+      T* dst = gg < p.E ? (T*)q.dw_a + (int64_t)gg * mn : (T*)q.dw_sh + (int64_t)(gg - p.E) * mn;
+      dw_reduce_block<DT>(q.partial + (int64_t)s_base[li] * mn, mn, nch, in ? b : b - b_in, dst);
+    }
+    __syncthreads();  // the list is read before the next round rewrites it
   }
 }
 

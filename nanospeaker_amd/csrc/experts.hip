@@ -15,7 +15,7 @@
 //                the hidden h, the gate gradient), then dA1 @ W_in[g]^T from LDS into
 //                per-row dX rows (reduced by `combine`).
 //   dw           dW_in[g] = x^T dA1 and dW_out[g] = h^T (w * dout) over the group's rows,
-//                split into row chunks of DW_RC; groups with several chunks write fp32
+//                split into row chunks of p.dw_rc; groups with several chunks write fp32
 //                partials that dw_reduce sums in chunk order (deterministic, no atomics).
 //   bias_grad    per-group column sums for the optional biases.
 #include <algorithm>
@@ -686,28 +686,32 @@ __global__ void __launch_bounds__(NT) dw_kernel(ExpParams p) {
   constexpr int TA = Stager::TA, TB = Stager::TB;
   constexpr int STAGE = KCH * (TA + TB);
   __shared__ __attribute__((aligned(16))) char s_stage[2][STAGE];
-  __shared__ int s_tok[DW_RC];
+  __shared__ int s_tok[DW_RC_MAX];
   __shared__ int s_loc[3];
 
   const int d = p.d, H = p.H, twoH = 2 * p.H;
   const int Md = MODE == 0 ? d : H;
   const int Nd = MODE == 0 ? twoH : d;
   const int tn = (Nd + BNo - 1) / BNo, ntiles = ((Md + BMo - 1) / BMo) * tn;
-  const int item = xcd_remap(blockIdx.x, gridDim.x);
+  const int item = xcd_deal(blockIdx.x, gridDim.x, ntiles);  // a chunk's tiles on one XCD
   Located loc;
-  if (!locate(item, p.E + p.S, [&](int g) { return dw_chunks(rows_of(p, g)) * ntiles; },
-              [&](int g) {
-                const int c = dw_chunks(rows_of(p, g));
+  // Shared groups first: v < S is group E + v, the rest the routed groups in order.
+  auto group_of = [&](int v) { return v < p.S ? p.E + v : v - p.S; };
+  auto chunks_of = [&](int v) { return dw_chunks(rows_of(p, group_of(v)), p.dw_rc); };
+  if (!locate(item, p.E + p.S, [&](int v) { return chunks_of(v) * ntiles; },
+              [&](int v) {
+                const int c = chunks_of(v);
                 return c > 1 ? c : 0;
               },
               s_loc, loc))
     return;
-  const int g = loc.g;
+  const int g = group_of(loc.g);
   const int rows_g = rows_of(p, g);
-  const int nch = dw_chunks(rows_g);
+  const int nch = dw_chunks(rows_g, p.dw_rc);
   const int chunk = loc.local / ntiles, t = loc.local % ntiles;
   const int m0 = (t / tn) * BMo, n0 = (t % tn) * BNo;
-  const int r0 = chunk * DW_RC, r1 = min(rows_g, r0 + DW_RC);
+  const int per = dw_chunk_rows(rows_g, nch);
+  const int r0 = min(rows_g, chunk * per), r1 = min(rows_g, r0 + per);
   const int64_t rs = row_start(p, g);
   const bool fast = p.fast;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lc = lane & 15, lg = lane >> 4;
@@ -789,30 +793,35 @@ __global__ void __launch_bounds__(NT) dw_kernel(ExpParams p) {
       }
 }
 
-// The dW split-K reduce (dw_reduce.h): one group per grid row, or both modes over the
-// multi-chunk groups in one launch.  grid = (dwr_blocks, rows).
-template <int DT, int MODE>
-__global__ void __launch_bounds__(NT) dw_reduce_kernel(ExpParams p) {
-  dw_reduce_group<DT, MODE>(p, blockIdx.y, blockIdx.x, gridDim.x);
-}
-
+// The dW split-K reduce (dw_reduce.h) as a launch of its own.
 template <int DT>
-__global__ void __launch_bounds__(NT) dw_reduce_pair_kernel(DwReduceArgs r) {
-  dw_reduce_pair_row<DT>(r, blockIdx.x, blockIdx.y);
+__global__ void __launch_bounds__(NT) dw_reduce_kernel(DwReduceArgs r) {
+  dw_reduce_wg<DT>(r, blockIdx.x);
 }
 
-// Rows of routed groups in dw_reduce_pair_kernel's grid: one per routed group when an
-// average routed group comes near a chunk (many of them then have several), else one row
-// for all of them.
-static int dw_reduce_routed_rows(const nsmoe_experts_args* a) {
-  return a->n_tokens * a->top_k > (int64_t)a->n_experts * (DW_RC * 9 / 10) ? a->n_experts : 1;
+// Rows per dW chunk: a thirty-sixth of all rows, a multiple of 32.  A chunk longer than that
+// is an item that outlasts the launch's other work; a shorter one splits more groups, and
+// every chunk of a split group writes an fp32 partial of 885 KB (d 576, H 128) that the
+// reduce reads again.  Measured training steps (us; 76 + 2 experts, top-6; rows in brackets)
+// by chunk length, balanced routing unless noted:
+//   T 2047 (16 k)           512: 159   768: 159   1536: 166   3072: 173
+//   T 8192 (66 k)           768: 287   1536: 281  2048: 279   3072: 293
+//   T 16384 (131 k)         768: 649   1536: 495  2048: 492   3072: 492   8192: 548
+//   T 16384, Zipf           1536: 534  3072: 528  8192: 583
+// (768 at T 16384 cuts every routed group in two: 134 MB of partials written and read.)
+// Below 512 rows a chunk is a few k-steps and the item's own setup dominates; 8192 is what
+// the items' token table in LDS holds.
+static int64_t dw_rows_per_chunk(const nsmoe_experts_args* a) {
+  const int64_t rows = a->n_tokens * (a->top_k + a->n_shared);
+  return std::clamp<int64_t>(cdiv(rows, 36 * 32) * 32, DW_RC_MIN, DW_RC_MAX);
 }
 
-// Workgroups per group of the dW reduce: one 16-byte vector of the larger dW per thread,
-// so every thread issues its chunk loads once.
-static unsigned dwr_blocks(const nsmoe_experts_args* a) {
-  const int64_t big = (int64_t)a->d_model * 2 * a->d_hidden;  // dW_in, the larger of the two
-  return (unsigned)std::min<int64_t>(cdiv(cdiv(big, 4), NT), 1024);
+// Workgroups of the dW reduce: one per (group, mode, block) item of the shared groups and of
+// two routed ones; more multi-chunk groups than that are taken in turn.
+static int dw_reduce_wgs(const nsmoe_experts_args* a) {
+  const int64_t mn = (int64_t)a->d_model * a->d_hidden;
+  const int64_t per = dw_reduce_blocks(2 * mn) + dw_reduce_blocks(mn);
+  return (int)std::min<int64_t>((a->n_shared + 2) * per, 4096);
 }
 
 // Bias gradients: WHICH 0 -> db_in[g] = sum_r dA1[slot_r]; 1 -> db_out[g] = sum_r w_r dout[tok_r].
@@ -915,6 +924,7 @@ static ExpParams make_params(const nsmoe_experts_args* a) {
   p.S = a->n_shared;
   p.k = a->top_k;
   p.act = a->activation;
+  p.dw_rc = (int)dw_rows_per_chunk(a);
   // Weight fragments and staged rows read 8 (2-byte types) or 4..8 (fp32) contiguous
   // elements per lane: the vector paths need d and H to be multiples of 8.
   p.fast = (a->d_model % 8 == 0) && (a->d_hidden % 8 == 0) && aligned16(a->x) &&
@@ -931,14 +941,14 @@ static int64_t fwd_grid(const nsmoe_experts_args* a) {
   return cdiv(M, BM) + nonempty + (int64_t)a->n_shared * cdiv(a->n_tokens, BM);
 }
 
-static int64_t dw_groups_chunks(const nsmoe_experts_args* a) {
-  const int64_t M = a->n_tokens * a->top_k;
-  return a->n_experts + cdiv(M, DW_RC) + (int64_t)a->n_shared * (cdiv(a->n_tokens, DW_RC) + 1);
+// Upper bound on the routed groups' chunks (an empty group has one).
+static int64_t dw_routed_chunks(const nsmoe_experts_args* a) {
+  return a->n_experts + cdiv(a->n_tokens * a->top_k, dw_rows_per_chunk(a));
 }
 
 static int64_t dw_partial_chunks(const nsmoe_experts_args* a) {
-  const int64_t M = a->n_tokens * a->top_k;
-  return 2 * cdiv(M, DW_RC) + 1 + (int64_t)a->n_shared * (cdiv(a->n_tokens, DW_RC) + 1);
+  const int64_t M = a->n_tokens * a->top_k, rc = dw_rows_per_chunk(a);
+  return 2 * cdiv(M, rc) + 1 + (int64_t)a->n_shared * cdiv(a->n_tokens, rc);
 }
 
 template <int DT>
@@ -1030,7 +1040,6 @@ static int experts_dw(const nsmoe_experts_args* a, const ExpParams& p,
                       hipStream_t s, DwReduceArgs* defer) {
   const int G = a->n_experts + a->n_shared;
   const int d = a->d_model, H = a->d_hidden;
-  const int64_t gc = dw_groups_chunks(a);
   ExpParams q_in = p, q_out = p;
   q_in.dw_a = gr->dw_in;
   q_in.dw_sh = gr->dw_sh_in;
@@ -1038,18 +1047,11 @@ static int experts_dw(const nsmoe_experts_args* a, const ExpParams& p,
   q_out.dw_a = gr->dw_out;
   q_out.dw_sh = gr->dw_sh_out;
   q_out.partial = (float*)(ws + L.p_out);
-  const int prc = launch_dw_pair_async(DT, q_in, q_out, gc, s);
+  const int prc = launch_dw_pair_async(DT, q_in, q_out, dw_routed_chunks(a), s);
   if (prc != -1) {
     NSMOE_TRY(prc);
-    const int rr = dw_reduce_routed_rows(a);
-    const DwReduceArgs r{q_in, q_out, rr, (int)dwr_blocks(a), 2 * (a->n_shared + rr)};
-    if (defer) {  // the caller's later launch runs it
-      *defer = r;
-    } else {
-      dw_reduce_pair_kernel<DT><<<dim3((unsigned)r.nbx, (unsigned)r.rows), NT, 0, s>>>(r);
-      NSMOE_TRY(check_launch("dw_reduce_pair_kernel"));
-    }
   } else {
+    const int64_t gc = dw_routed_chunks(a) + (int64_t)a->n_shared * dw_chunks((int)a->n_tokens, p.dw_rc);
     {  // dW_in
       const ExpParams& q = q_in;
       const int64_t ntiles = cdiv(d, 64) * cdiv(2 * H, 128);
@@ -1057,9 +1059,6 @@ static int experts_dw(const nsmoe_experts_args* a, const ExpParams& p,
       dw_kernel<DT, 0><<<(unsigned)(gc * ntiles), NT, 0, s>>>(q);
       timer.stop();
       NSMOE_TRY(check_launch("dw_kernel<in>"));
-      dim3 rg(dwr_blocks(a), (unsigned)G);
-      dw_reduce_kernel<DT, 0><<<rg, NT, 0, s>>>(q);
-      NSMOE_TRY(check_launch("dw_reduce_kernel<in>"));
     }
     {  // dW_out
       const ExpParams& q = q_out;
@@ -1068,10 +1067,14 @@ static int experts_dw(const nsmoe_experts_args* a, const ExpParams& p,
       dw_kernel<DT, 1><<<(unsigned)(gc * ntiles), NT, 0, s>>>(q);
       timer.stop();
       NSMOE_TRY(check_launch("dw_kernel<out>"));
-      dim3 rg(dwr_blocks(a), (unsigned)G);
-      dw_reduce_kernel<DT, 1><<<rg, NT, 0, s>>>(q);
-      NSMOE_TRY(check_launch("dw_reduce_kernel<out>"));
     }
+  }
+  const DwReduceArgs r{q_in, q_out, dw_reduce_wgs(a)};
+  if (defer) {  // the caller's later launch runs it
+    *defer = r;
+  } else {
+    dw_reduce_kernel<DT><<<(unsigned)r.wgs, NT, 0, s>>>(r);
+    NSMOE_TRY(check_launch("dw_reduce_kernel"));
   }
   if (gr->db_in || gr->db_sh_in) {
     ExpParams q = p;
@@ -1129,7 +1132,7 @@ static int experts_bwd_impl(const nsmoe_experts_args* a, const int32_t* inv, con
   hipStream_t s2 = side_fork(s, kSideSlotDw);
   // The reduce is handed to the caller only while dW runs on s itself (its partials are
   // then complete before any later launch on s).
-  if (defer) defer->nbx = 0;
+  if (defer) defer->wgs = 0;
   int rc = experts_dw<DT>(a, p, gr, ws, L, s2, s2 == s ? defer : nullptr);
   if (rc == NSMOE_OK && arc != -1) rc = launch_bwd_async(DT, p, nbw, grid, 1, s);
   if (rc == NSMOE_OK && combine)

@@ -1765,13 +1765,16 @@ struct DwLds {
   static_assert(STAGE == Geo<DT>::KC * (DwTile<1>::BMT + DwTile<1>::BNT) * 2,
                 "both modes stage the same bytes per step");
   char ring[S][STAGE];
-  int tok[DW_RC];
+  int tok[DW_RC_MAX];
   int loc[3];
 };
 
-// One (group, row chunk, output tile) item of dW; `item` indexes the mode's item space.
+// One (group, row chunk, output tile) item of dW; `item` indexes the mode's items of the
+// shared groups (their chunk counts follow from T) or of the routed ones (located from the
+// routing counts).
 template <int DT, int MODE, int S>
-__device__ __forceinline__ void dw_item(const ExpParams& p, int item, DwLds<DT, S>& L) {
+__device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int item,
+                                        DwLds<DT, S>& L) {
   using G = Geo<DT>;
   using T = typename G::T;
   using M = Mma<DT>;
@@ -1797,20 +1800,30 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, int item, DwLds<DT, 
   const int Md = MODE == 0 ? d : H;
   const int Nd = MODE == 0 ? twoH : d;
   const int tn = (Nd + BNT - 1) / BNT, ntiles = ((Md + BMT - 1) / BMT) * tn;
-  Located loc;
-  if (!locate(item, p.E + p.S, [&](int g) { return dw_chunks(rows_of(p, g)) * ntiles; },
-              [&](int g) {
-                const int c = dw_chunks(rows_of(p, g));
-                return c > 1 ? c : 0;
-              },
-              s_loc, loc))
-    return;
+  Located loc;  // aux: the group's first partial
+  if (shared) {
+    const int per = dw_chunks((int)p.T, p.dw_rc) * ntiles;
+    if (item >= p.S * per) return;
+    loc.g = p.E + item / per;
+    loc.local = item % per;
+    loc.aux = (item / per) * (per / ntiles);
+  } else {
+    if (!locate(item, p.E, [&](int g) { return dw_chunks(p.counts[g], p.dw_rc) * ntiles; },
+                [&](int g) {
+                  const int c = dw_chunks(p.counts[g], p.dw_rc);
+                  return c > 1 ? c : 0;
+                },
+                s_loc, loc))
+      return;
+    loc.aux += dw_shared_partials(p);
+  }
   const int g = loc.g;
   const int rows_g = rows_of(p, g);
-  const int nch = dw_chunks(rows_g);
+  const int nch = dw_chunks(rows_g, p.dw_rc);
   const int chunk = loc.local / ntiles, t = loc.local % ntiles;
   const int m0 = (t / tn) * BMT, n0 = (t % tn) * BNT;
-  const int r0 = chunk * DW_RC, nr = max(0, min(rows_g, r0 + DW_RC) - r0);
+  const int r0 = chunk * dw_chunk_rows(rows_g, nch);
+  const int nr = max(0, min(rows_g - r0, dw_chunk_rows(rows_g, nch)));
   const int64_t rs = row_start(p, g) + r0;
   const int tid = threadIdx.x, lane = tid & 63, lc = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1963,41 +1976,54 @@ __device__ __forceinline__ int dw_run(const ExpParams& p) {
   return ((Md + Tl::BMT - 1) / Tl::BMT) * ((Nd + Tl::BNT - 1) / Tl::BNT);
 }
 
-// dW_in and dW_out items in one launch: blocks [0, grid_in) take dW_in items, the rest
-// dW_out items (each part dealt over the XCDs on its own; grid_in is a multiple of 8 so
-// that block b - grid_in sits on the same XCD as b).  One launch fills the machine's
-// workgroup slots with both item sets instead of leaving a nearly empty round after each.
+// dW_in and dW_out items in one launch, in four parts, each dealt over the XCDs on its own
+// (every part is a multiple of 8 blocks, so a part's block b sits on XCD b % 8): the shared
+// groups' items of both modes first -- the longest -- then the routed groups'.  One launch
+// fills the machine's workgroup slots with every item instead of leaving a nearly empty
+// round after each.
+struct DwGrid {
+  int end[4];  // last block + 1 of: shared dW_in, shared dW_out, routed dW_in, routed dW_out
+};
+
 template <int DT, int S>
 __global__ void __launch_bounds__(NT, 2) dw_pair_kernel(ExpParams p_in, ExpParams p_out,
-                                                        int grid_in) {
+                                                        DwGrid gr) {
   __shared__ __attribute__((aligned(1024))) DwLds<DT, S> lds;
   const int b = blockIdx.x;
-  if (b < grid_in) dw_item<DT, 0, S>(p_in, xcd_deal(b, grid_in, dw_run<0>(p_in)), lds);
-  else
-    dw_item<DT, 1, S>(p_out, xcd_deal(b - grid_in, (int)gridDim.x - grid_in, dw_run<1>(p_out)),
-                      lds);
+  const int part = (b >= gr.end[0]) + (b >= gr.end[1]) + (b >= gr.end[2]);
+  const int b0 = part ? gr.end[part - 1] : 0, n = gr.end[part] - b0;
+  if (part & 1) dw_item<DT, 1, S>(p_out, part < 2, xcd_deal(b - b0, n, dw_run<1>(p_out)), lds);
+  else dw_item<DT, 0, S>(p_in, part < 2, xcd_deal(b - b0, n, dw_run<0>(p_in)), lds);
 }
 
 int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_out,
-                         int64_t groups_chunks, hipStream_t s) {
+                         int64_t routed_chunks, hipStream_t s) {
   if (!q_in.fast || (dtype != DT_BF16 && dtype != DT_F16)) return -1;
   if (q_in.T * q_in.d >= (int64_t(1) << 31)) return -1;  // token offsets are int32
   const int d = q_in.d, H = q_in.H;
-  // Rounded up to whole XCD rounds (the extra items are past the last real one and exit).
-  const int64_t g_in =
-      cdiv(groups_chunks * cdiv(d, DwTile<0>::BMT) * cdiv(2 * H, DwTile<0>::BNT), 8) * 8;
-  const int64_t g_out = groups_chunks * cdiv(H, DwTile<1>::BMT) * cdiv(d, DwTile<1>::BNT);
-  if (g_in + g_out <= 0) return NSMOE_OK;
+  const int64_t shared_chunks = (int64_t)q_in.S * dw_chunks((int)q_in.T, q_in.dw_rc);
+  const int64_t t_in = cdiv(d, DwTile<0>::BMT) * cdiv(2 * H, DwTile<0>::BNT);
+  const int64_t t_out = cdiv(H, DwTile<1>::BMT) * cdiv(d, DwTile<1>::BNT);
+  DwGrid gr;
+  int64_t end = 0;
+  const int64_t items[4] = {shared_chunks * t_in, shared_chunks * t_out, routed_chunks * t_in,
+                            routed_chunks * t_out};
+  for (int i = 0; i < 4; ++i) {
+    end += cdiv(items[i], 8) * 8;  // whole XCD rounds: the extra items exit at once
+    NSMOE_REQUIRE(end < INT32_MAX, "dW: too many items");
+    gr.end[i] = (int)end;
+  }
+  if (end <= 0) return NSMOE_OK;
   // Ring stages: 2 (one step of copies in flight, two workgroups per CU), which
   // measured ~1% faster per training step than 3; the "dw_stages" option asks for 3 or 4.
   const int st = option(OPT_DW_STAGES) ? (int)option(OPT_DW_STAGES) : 2;
   KernelTimer timer("dw", s);
-  const unsigned grid = (unsigned)(g_in + g_out);
+  const unsigned grid = (unsigned)end;
   auto go = [&](auto dt_tag) {
     constexpr int DT = decltype(dt_tag)::value;
-    if (st == 3) dw_pair_kernel<DT, 3><<<grid, NT, 0, s>>>(q_in, q_out, (int)g_in);
-    else if (st == 4) dw_pair_kernel<DT, 4><<<grid, NT, 0, s>>>(q_in, q_out, (int)g_in);
-    else dw_pair_kernel<DT, 2><<<grid, NT, 0, s>>>(q_in, q_out, (int)g_in);
+    if (st == 3) dw_pair_kernel<DT, 3><<<grid, NT, 0, s>>>(q_in, q_out, gr);
+    else if (st == 4) dw_pair_kernel<DT, 4><<<grid, NT, 0, s>>>(q_in, q_out, gr);
+    else dw_pair_kernel<DT, 2><<<grid, NT, 0, s>>>(q_in, q_out, gr);
   };
   if (dtype == DT_BF16) go(std::integral_constant<int, DT_BF16>{});
   else go(std::integral_constant<int, DT_F16>{});

@@ -8,7 +8,7 @@ namespace nsmoe {
 
 constexpr int BM = 64;      // rows per tile
 constexpr int NT = 256;     // threads per workgroup
-constexpr int DW_RC = 768;  // rows per dW chunk (work items of similar size)
+constexpr int DW_RC_MIN = 512, DW_RC_MAX = 8192;  // rows per dW chunk (dw_rows_per_chunk)
 constexpr int NP2 = 192;  // output columns per pass of the second GEMMs
 constexpr int XCD_RUN = 16;  // default tiles per XCD run of the token-tile kernels
 
@@ -54,6 +54,7 @@ struct ExpParams {
   void* dw_a;      // dW_in or dW_out (routed)
   void* dw_sh;     // shared counterpart
   float* partial;  // fp32 partials
+  int dw_rc;       // rows per dW chunk (dw_rows_per_chunk)
   void* db;        // bias grad (routed)
   void* db_sh;     // bias grad (shared)
 };
@@ -131,10 +132,23 @@ __device__ __forceinline__ void copy_out(const char* tile, int pitch, int rows,
 }
 
 
-// Row chunks of group g in the dW work decomposition.
-__device__ __forceinline__ int dw_chunks(int rows) {
-  const int c = (rows + DW_RC - 1) / DW_RC;
+// Row chunks of a group of `rows` rows in the dW work decomposition.
+__host__ __device__ __forceinline__ int dw_chunks(int rows, int rc) {
+  const int c = (rows + rc - 1) / rc;
   return c < 1 ? 1 : c;  // an empty group still owns one (all-zero) chunk
+}
+
+// Rows of each of a group's nch chunks (the last may have fewer): even shares, rounded up to
+// whole 32-row steps, at most the rows per chunk that nch was counted with.
+__device__ __forceinline__ int dw_chunk_rows(int rows, int nch) {
+  return ((rows + nch - 1) / nch + 31) & ~31;
+}
+
+// Partials (fp32 dW chunks) lie shared groups first, each a multi-chunk group's chunks in
+// order: the chunks of all shared groups, which routed group 0's follow.
+__device__ __forceinline__ int dw_shared_partials(const ExpParams& p) {
+  const int c = dw_chunks((int)p.T, p.dw_rc);
+  return c > 1 ? p.S * c : 0;
 }
 
 // Async (direct-to-LDS) variants for 16-bit types and d_hidden <= 128; each returns
@@ -142,7 +156,7 @@ __device__ __forceinline__ int dw_chunks(int rows) {
 int launch_fwd_async(int dtype, const ExpParams& p, int nbw, int64_t grid, hipStream_t s);
 // Both dW modes in one launch (q_in: dW_in, q_out: dW_out pointers and partials).
 int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_out,
-                         int64_t groups_chunks, hipStream_t s);
+                         int64_t routed_chunks, hipStream_t s);
 // Backward tiles: part 0 the GLU backward (fills p.da1, p.hbuf and p.dtw), part 1 the dX
 // rows from p.da1 (fills p.dxrow).  Both parts take or refuse the same shapes.
 int launch_bwd_async(int dtype, const ExpParams& p, int nbw, int64_t grid, int part,
@@ -163,8 +177,8 @@ struct DwReduceArgs;  // dw_reduce.h
 // act_in: the forward's saved pre-activations (experts_fwd_launch's act_out), or NULL to
 // recompute them.
 // defer_reduce: when set and dW runs on `stream`, the dW split-K reduce is not launched
-// but described there (nbx > 0) for a later launch on the stream to run (combine_dx's);
-// nbx = 0 when it ran here.
+// but described there (wgs > 0) for a later launch on the stream to run (combine_dx's);
+// wgs = 0 when it ran here.
 int experts_bwd_launch(const ::nsmoe_experts_args* a, const int32_t* inv, const void* grad_out,
                        const ::nsmoe_experts_grads* grads, void* workspace,
                        size_t workspace_bytes, bool combine, hipStream_t stream,

@@ -96,7 +96,7 @@ inline int64_t router_dw_reduce_blocks(int d, int ep) { return cdiv((int64_t)d *
 // With `rdw` set, workgroups past the token tiles (blockIdx.x >= tx) are the router dW's
 // reduce instead: its fp32 partials summed in chunk order into W.grad, streaming beside
 // the combine rather than as a launch of its own.  Workgroups from wx on are the experts'
-// dW split-K reduce (dw_reduce.h) when dwr.nbx > 0: the token tiles cover about half of
+// dW split-K reduce (dw_reduce.h) when dwr.wgs > 0: the token tiles cover about half of
 // the CUs, and the reduce streams on the others instead of in a launch of its own.
 template <int DT, int KM>
 __global__ void __launch_bounds__(NT, KM <= 6 ? 4 : 3)
@@ -110,8 +110,7 @@ combine_dx_kernel(CombineDxArgs a, RouterDwArgs rdw, int rchunks, int tx, DwRedu
   __shared__ __attribute__((aligned(1024))) char s_w[4 * CDX_KS][1024];  // the W tile
   if ((int)blockIdx.x >= wx) {  // uniform: an experts' dW reduce workgroup
     const int64_t f = (int64_t)(blockIdx.x - wx) * gridDim.y + blockIdx.y;
-    const int y = (int)(f / dwr.nbx), bx = (int)(f - (int64_t)y * dwr.nbx);
-    if (y < dwr.rows) dw_reduce_pair_row<DT>(dwr, bx, y);
+    if (f < dwr.wgs) dw_reduce_wg<DT>(dwr, (int)f);
     return;
   }
   if ((int)blockIdx.x >= tx) {  // uniform: a router dW reduce workgroup
@@ -390,9 +389,9 @@ int combine_dx_launch(int dtype, const CombineDxArgs& a, const RouterDwArgs* rdw
   const int64_t tx = cdiv(a.T, CDX_TOK), ty = cdiv(a.d, CDX_COLS);
   const int64_t rx = rdw ? cdiv(router_dw_reduce_blocks(a.d, a.ep), ty) : 0;
   // The experts' dW reduce workgroups, flattened over the grid's columns.
-  const bool red = dwr && dwr->nbx > 0 && dwr->rows > 0;
+  const bool red = dwr && dwr->wgs > 0;
   const int64_t wx = tx + rx;
-  const int64_t dx_extra = red ? cdiv((int64_t)dwr->nbx * dwr->rows, ty) : 0;
+  const int64_t dx_extra = red ? cdiv(dwr->wgs, ty) : 0;
   NSMOE_REQUIRE(wx + dx_extra < INT32_MAX, "combine_dx: %lld tokens", (long long)a.T);
   const dim3 grid((unsigned)(wx + dx_extra), (unsigned)ty);
   DwReduceArgs dr{};

@@ -252,6 +252,18 @@ def test_zero_router_sends_every_token_to_the_same_experts():
     assert int((ref.counts > 0).sum()) == 6 and int(ref.counts.max()) == 2048
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [511, 512, 513, 1057])
+def test_dw_chunk_edges(T, dtype):
+    """The dW row chunks (512 rows at these sizes) at their edges: shared groups of one row
+    less than a chunk, exactly one, one more, and three chunks of even shares (353 -> 384
+    rows, the last one short), beside routed groups of one chunk (4 experts, top-1) and of
+    up to two (8 experts, top-4).  Only multi-chunk groups write partials; the reduce sums
+    them."""
+    run_case(T, train=True, backward=True, d=128, E=4, d_ff=96, k=1, S=2, dtype=dtype)
+    run_case(T, train=True, backward=True, d=128, E=8, d_ff=96, k=4, S=1, dtype=dtype)
+
+
 @pytest.mark.parametrize("cfg", [dict(S=2), dict(S=0, bias=True, dtype=torch.float16),
                                  dict(d=128, E=12, d_ff=96, k=4, S=1)])
 def test_saved_pre_activations_and_recompute_agree(monkeypatch, cfg):
