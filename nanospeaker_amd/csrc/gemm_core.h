@@ -19,6 +19,8 @@
 //     the staging stores and the 16-lane fragment reads touch distinct banks.
 #pragma once
 
+#include <type_traits>
+
 #include "nsmoe_common.h"
 
 namespace nsmoe {
@@ -75,6 +77,34 @@ template <> struct Mma<DT_F32> {
                                                  __uint_as_float(b.hi[i]), acc, 0, 0, 0);
   }
 };
+
+// acc[i][j] += a[i] b[j] over one 32-element k step, for the first `rows` row blocks.  fp32
+// issues its eight 4-element MFMAs block by block, so that consecutive ones write different
+// accumulators (each accumulator still adds its k elements in order).
+template <int DT, int NA, int NB>
+__device__ __forceinline__ void mma_tile(f32x4 (&acc)[NA][NB], const typename Mma<DT>::Frag* a,
+                                         const typename Mma<DT>::Frag* b, int rows) {
+  if constexpr (DT == DT_F32) {
+    auto part = [&](auto n_tag) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < decltype(n_tag)::value; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                __uint_as_float(e < 4 ? a[i].lo[e & 3] : a[i].hi[e & 3]),
+                __uint_as_float(e < 4 ? b[j].lo[e & 3] : b[j].hi[e & 3]), acc[i][j], 0, 0, 0);
+    };
+    if (rows == 1) part(std::integral_constant<int, 1>{});
+    else part(std::integral_constant<int, NA>{});
+  } else {
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < NA; ++i) Mma<DT>::run(acc[i][j], a[i], b[j]);
+  }
+}
 
 // ---- swizzled 32-element LDS rows ---------------------------------------------------------
 //

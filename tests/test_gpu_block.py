@@ -264,6 +264,15 @@ def test_dw_chunk_edges(T, dtype):
     run_case(T, train=True, backward=True, d=128, E=8, d_ff=96, k=4, S=1, dtype=dtype)
 
 
+@pytest.mark.parametrize("T", [1, 15, 17, 31, 33, 49])
+def test_fp32_tile_edges(T):
+    """fp32's 32-row tiles: groups of every remainder of a tile (the shared groups hold all T
+    tokens, the routed ones a few), tiles of one 16-row block and of two, and d and H that
+    end inside a fragment and inside a pass of 192 columns."""
+    run_case(T, train=True, backward=True, dtype=torch.float32, d=200, E=6, d_ff=60, k=2, S=2)
+    run_case(T, train=True, backward=True, dtype=torch.float32, d=576, E=4, d_ff=192, k=2, S=1)
+
+
 @pytest.mark.parametrize("cfg", [dict(S=2), dict(S=0, bias=True, dtype=torch.float16),
                                  dict(d=128, E=12, d_ff=96, k=4, S=1)])
 def test_saved_pre_activations_and_recompute_agree(monkeypatch, cfg):
