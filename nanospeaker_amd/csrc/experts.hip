@@ -406,7 +406,9 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
       const int jb = wave * NBW + j;
       b[j] = frag_pk<DT>(P1, jb, kb, p.in_kb);
       b[NBW + j] = frag_pk<DT>(P1, HPMAX / 16 + jb, kb, p.in_kb);
-      b[2 * NBW + j] = frag_rows<DT>(rowWo, jb * 16, kb * G::KC, d, fast);
+      if constexpr (DT == DT_F32)
+        b[2 * NBW + j] = frag_rows_quads(rowWo, jb * 16, kb * G::KC, d, fast);
+      else b[2 * NBW + j] = frag_rows<DT>(rowWo, jb * 16, kb * G::KC, d, fast);
     }
   };
   const int nk = p.in_kb;
@@ -421,10 +423,18 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
 #pragma unroll
     for (int i = 0; i < MR; ++i) {
       ax[i] = frag_sw<DT>(s_ax[kc & 1], i * 16);
-      ad[i] = frag_sw<DT>(s_ad[kc & 1], i * 16);
+      if constexpr (DT == DT_F32) ad[i] = frag_sw_halves(s_ad[kc & 1], i * 16);
+      else ad[i] = frag_sw<DT>(s_ad[kc & 1], i * 16);
     }
     mma_tile<DT>(acc1, ax, use, rb);
-    mma_tile<DT>(accG, ad, use + 2 * NBW, rb);
+    if constexpr (DT == DT_F32) {
+      Frag wo[NBW];
+#pragma unroll
+      for (int j = 0; j < NBW; ++j) wo[j] = frag_from_quads(use[2 * NBW + j]);
+      mma_tile<DT>(accG, ad, wo, rb);
+    } else {
+      mma_tile<DT>(accG, ad, use + 2 * NBW, rb);
+    }
     if (more) {
       stX.store(s_ax[(kc + 1) & 1]);
       stD.store(s_ad[(kc + 1) & 1]);
@@ -528,7 +538,9 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
       const int half = q / nkh, kk = (q % nkh) * G::KC;
 #pragma unroll
       for (int j = 0; j < 3; ++j)
-        b[j] = frag_rows<DT>(rowWi, nw + j * 16, half * H + kk, half * H + H, fast);
+        if constexpr (DT == DT_F32)
+          b[j] = frag_rows_quads(rowWi, nw + j * 16, half * H + kk, half * H + H, fast);
+        else b[j] = frag_rows<DT>(rowWi, nw + j * 16, half * H + kk, half * H + H, fast);
     };
     Frag c0[3], c1[3];
     loadB3(c0, 0);
@@ -540,8 +552,18 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
       const int kbyte = (half * HPMAX + kk) * G::ES;
       Frag af[MR];
 #pragma unroll
-      for (int i = 0; i < MR; ++i) af[i] = frag_at<DT>(s_da, DA_PITCH, i * 16, kbyte);
-      mma_tile<DT>(acc, af, use, rb);
+      for (int i = 0; i < MR; ++i) {
+        if constexpr (DT == DT_F32) af[i] = frag_at_halves(s_da, DA_PITCH, i * 16, kbyte);
+        else af[i] = frag_at<DT>(s_da, DA_PITCH, i * 16, kbyte);
+      }
+      if constexpr (DT == DT_F32) {
+        Frag wi[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) wi[j] = frag_from_quads(use[j]);
+        mma_tile<DT>(acc, af, wi, rb);
+      } else {
+        mma_tile<DT>(acc, af, use, rb);
+      }
     }
 #pragma unroll
     for (int j = 0; j < 3; ++j) {

@@ -1744,8 +1744,15 @@ int launch_bwd_async(int dtype, const ExpParams& p, int nbw, int64_t grid, int p
 //
 // Chunk swizzle: a transpose read of one fragment touches 2 chunks (32 B) of each of 4
 // rows per 16 lanes; the swizzle spreads the 8 rows a half-wave reads over all 64 banks.
-template <int ROWB>
+//
+// fp32 operands are read a float a lane, 16 columns (4 chunks) of 4 rows at a time: the
+// swizzle puts the 4 rows on the 4 quarters of the banks.
+template <int DT, int ROWB>
 __device__ __forceinline__ int dw_swz(int r) {
+  if constexpr (Geo<DT>::ES == 4) {
+    static_assert(ROWB % 256 == 0, "rows of whole 256-byte lines");
+    return (r & 3) << 2;
+  }
   static_assert(ROWB % 128 == 0, "rows of whole 128-byte lines");
   if constexpr (ROWB % 256 == 0) return ((r & 3) | (((r >> 3) & 1) << 2)) << 1;
   else return (((r >> 1) ^ (r >> 2)) & 3) << 1;
@@ -1759,10 +1766,15 @@ template <> struct DwTile<1> {  // dW_out [H, d]: 128 x 192 tiles
   static constexpr int BMT = 128, BNT = 192, WM = 2, WN = 2;
 };
 
+// Rows per k-step: 32 of 16-bit elements, 16 of fp32 (the same bytes).
+template <int DT>
+constexpr int dw_step_rows() { return 64 / Geo<DT>::ES; }
+
 template <int DT, int S>
 struct DwLds {
-  static constexpr int STAGE = Geo<DT>::KC * (DwTile<0>::BMT + DwTile<0>::BNT) * 2;
-  static_assert(STAGE == Geo<DT>::KC * (DwTile<1>::BMT + DwTile<1>::BNT) * 2,
+  static constexpr int STAGE =
+      dw_step_rows<DT>() * (DwTile<0>::BMT + DwTile<0>::BNT) * Geo<DT>::ES;
+  static_assert(STAGE == dw_step_rows<DT>() * (DwTile<1>::BMT + DwTile<1>::BNT) * Geo<DT>::ES,
                 "both modes stage the same bytes per step");
   char ring[S][STAGE];
   int tok[DW_RC_MAX];
@@ -1780,12 +1792,12 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
   using M = Mma<DT>;
   using Frag = typename M::Frag;
   using Tl = DwTile<MODE>;
-  static_assert(G::ES == 2, "16-bit types only");
   constexpr int BMT = Tl::BMT, BNT = Tl::BNT;
   constexpr int TMB = BMT / 16 / Tl::WM, TNB = BNT / 16 / Tl::WN;  // blocks per wave
-  constexpr int QROWB = BMT * 2, PROWB = BNT * 2;                 // LDS row bytes
-  constexpr int QCPR = BMT / 8, PCPR = BNT / 8;                   // 16-byte chunks per row
-  constexpr int QBYTES = G::KC * QROWB, PBYTES = G::KC * PROWB;
+  constexpr int KS = dw_step_rows<DT>();                          // rows per k-step
+  constexpr int QROWB = BMT * G::ES, PROWB = BNT * G::ES;         // LDS row bytes
+  constexpr int QCPR = QROWB / 16, PCPR = PROWB / 16;             // 16-byte chunks per row
+  constexpr int QBYTES = KS * QROWB, PBYTES = KS * PROWB;
   constexpr int QBLK = QBYTES / 1024, PBLK = PBYTES / 1024;       // 1 KiB copy blocks
   constexpr int STAGE = QBYTES + PBYTES;
   constexpr int NBLK = QBLK + PBLK;
@@ -1840,7 +1852,7 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
   const T* HB = (const T*)p.hbuf;
   const T* DO = (const T*)p.dout;
   const T* zero = (const T*)((const char*)g_zero_kib + lane * 16);
-  const int nsteps = (nr + G::KC - 1) / G::KC;
+  const int nsteps = (nr + KS - 1) / KS;
 
   // The copy plan, fixed for the item.  Copy u of this wave moves one 16-byte chunk of
   // the 1 KiB block b = 4u + wave: chunk column (swizzled on the source side) and row
@@ -1863,11 +1875,11 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
     bool ok;
     if (isq) {
       row = q / QCPR;
-      col = m0 + ((q % QCPR) ^ dw_swz<QROWB>(row)) * 8;
+      col = m0 + ((q % QCPR) ^ dw_swz<DT, QROWB>(row)) * G::VE;
       ok = col < Md;
     } else {
       row = q / PCPR;
-      col = n0 + ((q % PCPR) ^ dw_swz<PROWB>(row)) * 8;
+      col = n0 + ((q % PCPR) ^ dw_swz<DT, PROWB>(row)) * G::VE;
       ok = col < Nd;
     }
     crow[u] = ok ? row : (1 << 20);
@@ -1879,10 +1891,10 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
   auto read_tok = [&](int s) {
 #pragma unroll
     for (int u = 0; u < LOADS; ++u)
-      if (gathered(u)) ctok[u] = s_tok[s * G::KC + (crow[u] & 31)];
+      if (gathered(u)) ctok[u] = s_tok[s * KS + (crow[u] & (KS - 1))];
   };
   auto issue = [&](int s, int stage) {
-    const int k0 = s * G::KC;
+    const int k0 = s * KS;
     const uint32_t dst = ring + stage * STAGE + wave * 1024;
 #pragma unroll
     for (int u = 0; u < LOADS; ++u) {
@@ -1902,10 +1914,10 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
     const int col = col0 + 4 * (i & 3);
     const int c = col >> 3, cb = (col & 7) * 2;
     const int ra = 8 * gq + (i >> 2), rb = ra + 4;
-    const uint2 lo = lds_read_tr16(tile + ra * RB + ((c ^ dw_swz<RB>(ra)) << 4) + cb);
-    const uint2 hi = lds_read_tr16(tile + rb * RB + ((c ^ dw_swz<RB>(rb)) << 4) + cb);
+    const uint2 lo = lds_read_tr16(tile + ra * RB + ((c ^ dw_swz<DT, RB>(ra)) << 4) + cb);
+    const uint2 hi = lds_read_tr16(tile + rb * RB + ((c ^ dw_swz<DT, RB>(rb)) << 4) + cb);
     Frag f;
-    f.v = u32x4{lo.x, lo.y, hi.x, hi.y};
+    if constexpr (G::ES == 2) f.v = u32x4{lo.x, lo.y, hi.x, hi.y};
     return f;
   };
 
@@ -1922,17 +1934,42 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
     barrier_lds();
     if (s + S - 1 < nsteps) issue(s + S - 1, (ST + S - 1) % S);
     const char* st = L.ring[ST];
-    Frag qf[TMB], pf[TNB];
+    if constexpr (G::ES == 4) {
+      // lane 16 q + c of k sub-step e: row 4 e + q, column c of each block
+      auto elem = [&](const char* tile, auto rowb_tag, int col0, int e) -> float {
+        constexpr int RB = decltype(rowb_tag)::value;
+        const int row = 4 * e + lg, col = col0 + lc;
+        return *(const float*)(tile + row * RB + (((col >> 2) ^ dw_swz<DT, RB>(row)) << 4) +
+                               (col & 3) * 4);
+      };
 #pragma unroll
-    for (int i = 0; i < TMB; ++i)
-      qf[i] = frag_tr(st, std::integral_constant<int, QROWB>{}, (wm * TMB + i) * 16);
+      for (int e = 0; e < KS / 4; ++e) {
+        float q[TMB], pv[TNB];
 #pragma unroll
-    for (int j = 0; j < TNB; ++j)
-      pf[j] = frag_tr(st + QBYTES, std::integral_constant<int, PROWB>{}, (wn * TNB + j) * 16);
+        for (int i = 0; i < TMB; ++i)
+          q[i] = elem(st, std::integral_constant<int, QROWB>{}, (wm * TMB + i) * 16, e);
 #pragma unroll
-    for (int j = 0; j < TNB; ++j)
+        for (int j = 0; j < TNB; ++j)
+          pv[j] = elem(st + QBYTES, std::integral_constant<int, PROWB>{}, (wn * TNB + j) * 16, e);
 #pragma unroll
-      for (int i = 0; i < TMB; ++i) M::run(acc[j][i], pf[j], qf[i]);
+        for (int j = 0; j < TNB; ++j)
+#pragma unroll
+          for (int i = 0; i < TMB; ++i)
+            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(pv[j], q[i], acc[j][i], 0, 0, 0);
+      }
+    } else {
+      Frag qf[TMB], pf[TNB];
+#pragma unroll
+      for (int i = 0; i < TMB; ++i)
+        qf[i] = frag_tr(st, std::integral_constant<int, QROWB>{}, (wm * TMB + i) * 16);
+#pragma unroll
+      for (int j = 0; j < TNB; ++j)
+        pf[j] = frag_tr(st + QBYTES, std::integral_constant<int, PROWB>{}, (wn * TNB + j) * 16);
+#pragma unroll
+      for (int j = 0; j < TNB; ++j)
+#pragma unroll
+        for (int i = 0; i < TMB; ++i) M::run(acc[j][i], pf[j], qf[i]);
+    }
   };
   if (nsteps > 0) read_tok(0);
   for (int s = 0; s < S - 1 && s < nsteps; ++s) issue(s, s);
@@ -1959,10 +1996,10 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
       const int m = m0 + (wm * TMB + i) * 16 + lc;
       if (m >= Md) continue;
       const f32x4 v = acc[j][i];
-      if (dst)
-        *(uint2*)(dst + (int64_t)m * Nd + n) = make_uint2(pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3]));
+      if (pdst) *(f32x4*)(pdst + (int64_t)m * Nd + n) = v;
+      else if constexpr (G::ES == 4) *(f32x4*)(dst + (int64_t)m * Nd + n) = v;
       else
-        *(f32x4*)(pdst + (int64_t)m * Nd + n) = v;
+        *(uint2*)(dst + (int64_t)m * Nd + n) = make_uint2(pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3]));
     }
   }
 }
@@ -1998,7 +2035,7 @@ __global__ void __launch_bounds__(NT, 2) dw_pair_kernel(ExpParams p_in, ExpParam
 
 int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_out,
                          int64_t routed_chunks, hipStream_t s) {
-  if (!q_in.fast || (dtype != DT_BF16 && dtype != DT_F16)) return -1;
+  if (!q_in.fast) return -1;
   if (q_in.T * q_in.d >= (int64_t(1) << 31)) return -1;  // token offsets are int32
   const int d = q_in.d, H = q_in.H;
   const int64_t shared_chunks = (int64_t)q_in.S * dw_chunks((int)q_in.T, q_in.dw_rc);
@@ -2021,12 +2058,14 @@ int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_ou
   const unsigned grid = (unsigned)end;
   auto go = [&](auto dt_tag) {
     constexpr int DT = decltype(dt_tag)::value;
-    if (st == 3) dw_pair_kernel<DT, 3><<<grid, NT, 0, s>>>(q_in, q_out, gr);
+    if constexpr (DT == DT_F32) dw_pair_kernel<DT, 2><<<grid, NT, 0, s>>>(q_in, q_out, gr);
+    else if (st == 3) dw_pair_kernel<DT, 3><<<grid, NT, 0, s>>>(q_in, q_out, gr);
     else if (st == 4) dw_pair_kernel<DT, 4><<<grid, NT, 0, s>>>(q_in, q_out, gr);
     else dw_pair_kernel<DT, 2><<<grid, NT, 0, s>>>(q_in, q_out, gr);
   };
   if (dtype == DT_BF16) go(std::integral_constant<int, DT_BF16>{});
-  else go(std::integral_constant<int, DT_F16>{});
+  else if (dtype == DT_F16) go(std::integral_constant<int, DT_F16>{});
+  else go(std::integral_constant<int, DT_F32>{});
   timer.stop();
   return check_launch("dw_pair_kernel");
 }

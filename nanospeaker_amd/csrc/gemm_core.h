@@ -146,12 +146,14 @@ __device__ __forceinline__ typename Mma<DT>::Frag frag_at(const char* tile, int 
   return Mma<DT>::load(tile + (row0 + (l & 15)) * pitch + kbyte0 + (l >> 4) * Geo<DT>::FRAGB);
 }
 
-// Packed weight fragment (nb, kb) of a [n_blocks][k_blocks] fragment-order array.
+// Packed weight fragment (nb, kb) of a [n_blocks][k_blocks] fragment-order array: the lanes'
+// first 16 bytes, then (fp32) their second ones, so each load is one contiguous KiB.
 template <int DT>
 __device__ __forceinline__ typename Mma<DT>::Frag frag_pk(const char* pk, int nb, int kb,
                                                           int k_blocks) {
-  return Mma<DT>::load(pk + ((int64_t)nb * k_blocks + kb) * Geo<DT>::PKB +
-                       lane_id() * Geo<DT>::FRAGB);
+  const char* src = pk + ((int64_t)nb * k_blocks + kb) * Geo<DT>::PKB + lane_id() * 16;
+  if constexpr (Geo<DT>::ES == 2) return Mma<DT>::load(src);
+  else return typename Mma<DT>::Frag{*(const u32x4*)src, *(const u32x4*)(src + 1024)};
 }
 
 // Fragment of a row-major source whose rows are the fragment's 16 columns and whose k
@@ -294,6 +296,49 @@ __device__ __forceinline__ uint32_t bperm(int addr, uint32_t v) {
 }
 __device__ __forceinline__ u32x4 bperm4(int addr, const u32x4& v) {
   return u32x4{bperm(addr, v[0]), bperm(addr, v[1]), bperm(addr, v[2]), bperm(addr, v[3])};
+}
+
+// ---- fp32 row operands in the quad order ----
+//
+// A row-major fp32 operand (column n0 + r of the fragment is row(n0 + r), k contiguous, 32 of
+// them = 128 bytes) loaded quad-major -- lane 4 r + c takes 16-byte chunks c and 4 + c of row
+// r -- and moved to the MFMA order when it is used: lane 16 q + r then holds k elements
+// 4 q .. + 3 (lo) and 16 + 4 q .. + 3 (hi), an assignment that the other operand's reads
+// (frag_sw_halves, frag_at_halves) share.
+template <class RowPtr>
+__device__ __forceinline__ Mma<DT_F32>::Frag frag_rows_quads(RowPtr row, int n0, int k0, int klim,
+                                                             bool fast) {
+  const int l = lane_id();
+  const float* src = row(n0 + (l >> 2));
+  const int k = k0 + 4 * (l & 3);
+  Mma<DT_F32>::Frag f = Mma<DT_F32>::zero();
+  if (!src) return f;
+  if (fast) {  // klim % 4 == 0: a chunk is inside or outside
+    if (k < klim) f.lo = *(const u32x4*)(src + k);
+    if (k + 16 < klim) f.hi = *(const u32x4*)(src + k + 16);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f.lo[e] = k + e < klim ? __float_as_uint(src[k + e]) : 0u;
+      f.hi[e] = k + 16 + e < klim ? __float_as_uint(src[k + 16 + e]) : 0u;
+    }
+  }
+  return f;
+}
+__device__ __forceinline__ Mma<DT_F32>::Frag frag_from_quads(const Mma<DT_F32>::Frag& f) {
+  const int a = bperm_from_quads(lane_id());
+  return Mma<DT_F32>::Frag{bperm4(a, f.lo), bperm4(a, f.hi)};
+}
+__device__ __forceinline__ Mma<DT_F32>::Frag frag_sw_halves(const char* tile, int row0) {
+  const int l = lane_id(), r = row0 + (l & 15), q = l >> 4;
+  return Mma<DT_F32>::Frag{*(const u32x4*)(tile + sw_off<DT_F32>(r, q)),
+                           *(const u32x4*)(tile + sw_off<DT_F32>(r, 4 + q))};
+}
+__device__ __forceinline__ Mma<DT_F32>::Frag frag_at_halves(const char* tile, int pitch, int row0,
+                                                            int kbyte0) {
+  const int l = lane_id();
+  const char* src = tile + (row0 + (l & 15)) * pitch + kbyte0 + (l >> 4) * 16;
+  return Mma<DT_F32>::Frag{*(const u32x4*)src, *(const u32x4*)(src + 64)};
 }
 
 // Workgroup barrier for data that reached LDS by LDS-DMA copies the caller has already

@@ -6,6 +6,7 @@
 // columns, 32 contraction elements) of every (column block nb, k block kb) is one
 // contiguous block laid out exactly as the 64 lanes consume it:
 //   packed[g][nb][kb][lane][8]   lane = (k % 32) / 8 * 16 + n % 16,  element = k % 8
+// (fp32: [2][lane][4], the lanes' elements 0 .. 3, then 4 .. 7)
 // so the expert kernels load each weight fragment with one coalesced 16-byte-per-lane
 // load straight from L2, and never stage weights through LDS.
 //
@@ -58,8 +59,9 @@ pack_kernel(const typename Elem<DT>::T* __restrict__ routed,
   const int wave = threadIdx.x >> 6;
   const typename Mma<DT>::Frag f = frag_sw<DT>(tile, wave * 16);
   const int nb = nt * 4 + wave;
-  char* dst = out + (((int64_t)g * n_nb + nb) * n_kb + kb) * G::PKB + lane_id() * G::FRAGB;
-  __builtin_memcpy(dst, &f, sizeof(f));
+  char* dst = out + (((int64_t)g * n_nb + nb) * n_kb + kb) * G::PKB + lane_id() * 16;
+  *(u32x4*)dst = f.lo;
+  *(u32x4*)(dst + 1024) = f.hi;
 }
 
 // Both 16-bit packs in one launch (W_in alone when items_out is 0): every wave packs
