@@ -37,8 +37,59 @@ namespace nsmoe {
 // LDS and feeds GEMM2 [rows, H] x [H, d] against packed W_out in 192-column passes
 // (48 columns per wave); + b_out, * gate weight, then the rows go out through LDS.
 
+// acc += A B over nk k-steps of 32: A's rows (16 MR of them, `row`) staged through the two
+// swizzled LDS tiles s_a, B's fragments of step kb loaded by loadB(frags, kb).  16-bit types
+// hold two buffers of B fragments, loaded a step ahead; fp32 one, refilled behind its last
+// use -- three workgroups per CU then cover the loads, where two buffers left room for two.
+// QUADS (fp32): loadB loads quad-major (frag_rows_quads).
+template <int DT, int MR, int NB, bool QUADS, class RowPtr, class LoadB>
+__device__ __forceinline__ void k_loop(char (*s_a)[16 * MR * Geo<DT>::ROWB], RowPtr row,
+                                       LoadB loadB, int nk, int d, bool fast,
+                                       f32x4 (&acc)[MR][NB], int rb) {
+  using G = Geo<DT>;
+  using Frag = typename Mma<DT>::Frag;
+  constexpr bool ONE = DT == DT_F32;
+  DirectStage<DT, 16 * MR, NT> st;
+  Frag b0[NB], b1[ONE ? 1 : NB];
+  auto step = [&](int kc, Frag* use, Frag* nxt) {
+    const bool more = kc + 1 < nk;
+    if (more) {
+      st.load(row, (kc + 1) * G::KC, d, fast);
+      if (!ONE) loadB(nxt, kc + 1);
+    }
+    Frag af[MR];
+#pragma unroll
+    for (int i = 0; i < MR; ++i) {
+      if constexpr (QUADS) af[i] = frag_sw_halves(s_a[kc & 1], i * 16);
+      else af[i] = frag_sw<DT>(s_a[kc & 1], i * 16);
+    }
+    if constexpr (QUADS) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) use[j] = frag_from_quads(use[j]);
+    }
+    mma_tile<DT>(acc, af, use, rb);
+    if (more) {
+      if (ONE) loadB(nxt, kc + 1);
+      st.store(s_a[(kc + 1) & 1]);
+    }
+    __syncthreads();
+  };
+  st.load(row, 0, d, fast);
+  loadB(b0, 0);
+  st.store(s_a[0]);
+  __syncthreads();
+  if constexpr (ONE) {
+    for (int kc = 0; kc < nk; ++kc) step(kc, b0, b0);
+  } else {
+    for (int kc = 0; kc < nk; kc += 2) {
+      step(kc, b0, b1);
+      if (kc + 1 < nk) step(kc + 1, b1, b0);
+    }
+  }
+}
+
 template <int DT, int NBW, int MR>
-__global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_fwd_kernel(ExpParams p) {
+__global__ void __launch_bounds__(NT, DT == DT_F32 ? 3 : 1) expert_fwd_kernel(ExpParams p) {
   using G = Geo<DT>;
   using T = typename G::T;
   using M = Mma<DT>;
@@ -85,13 +136,12 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_fwd_kernel(Ex
   const char* P1 = p.p_in + (int64_t)g * p.in_nb * p.in_kb * G::PKB;
 
   // ---- GEMM1 ----
-  DirectStage<DT, RT, NT> stA;
+  constexpr bool ONE = DT == DT_F32;  // one buffer of weight fragments (k_loop)
   f32x4 acc1[MR][2 * NBW];  // gate blocks, then up blocks
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
     for (int j = 0; j < 2 * NBW; ++j) acc1[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Frag b0[2 * NBW], b1[2 * NBW];
   auto loadB = [&](Frag* b, int kb) {
 #pragma unroll
     for (int j = 0; j < NBW; ++j) {
@@ -100,28 +150,7 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_fwd_kernel(Ex
       b[NBW + j] = frag_pk<DT>(P1, HPMAX / 16 + jb, kb, p.in_kb);
     }
   };
-  const int nk = p.in_kb;
-  auto step = [&](int kc, const Frag* use, Frag* nxt) {
-    const bool more = kc + 1 < nk;
-    if (more) {
-      stA.load(rowA, (kc + 1) * G::KC, d, fast);
-      loadB(nxt, kc + 1);
-    }
-    Frag af[MR];
-#pragma unroll
-    for (int i = 0; i < MR; ++i) af[i] = frag_sw<DT>(s_a[kc & 1], i * 16);
-    mma_tile<DT>(acc1, af, use, rb);
-    if (more) stA.store(s_a[(kc + 1) & 1]);
-    __syncthreads();
-  };
-  stA.load(rowA, 0, d, fast);
-  loadB(b0, 0);
-  stA.store(s_a[0]);
-  __syncthreads();
-  for (int kc = 0; kc < nk; kc += 2) {
-    step(kc, b0, b1);
-    if (kc + 1 < nk) step(kc + 1, b1, b0);
-  }
+  k_loop<DT, MR, 2 * NBW, false>(s_a, rowA, loadB, p.in_kb, d, fast, acc1, rb);
 
   // ---- GEMM1 epilogue: bias, h = act(gate) * up into LDS ----
   const T* bin = (g < p.E ? p.b_in : p.b_sh_in)
@@ -165,13 +194,14 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_fwd_kernel(Ex
     Frag c0[3], c1[3];
     loadB2(c0, 0);
     for (int kk = 0; kk < nk2; ++kk) {
-      Frag* use = (kk & 1) ? c1 : c0;
-      Frag* nxt = (kk & 1) ? c0 : c1;
-      if (kk + 1 < nk2) loadB2(nxt, kk + 1);
+      Frag* use = !ONE && (kk & 1) ? c1 : c0;
+      Frag* nxt = ONE || (kk & 1) ? c0 : c1;
+      if (!ONE && kk + 1 < nk2) loadB2(nxt, kk + 1);
       Frag af[MR];
 #pragma unroll
       for (int i = 0; i < MR; ++i) af[i] = frag_at<DT>(s_h, HP_PITCH, i * 16, kk * G::ROWB);
       mma_tile<DT>(acc, af, use, rb);
+      if (ONE && kk + 1 < nk2) loadB2(nxt, kk + 1);
     }
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
@@ -317,7 +347,8 @@ combine_kernel(const typename Elem<DT>::T* __restrict__ rows, const int32_t* __r
 
 // ============================ backward: recompute, GLU backward, dX rows ==================
 //
-// Phase 1 runs three GEMMs over the same 16 MR gathered token rows and K = d in one loop:
+// Phase 1 runs three GEMMs over the same 16 MR gathered token rows and K = d, a1 in one loop
+// and G in the next (fewer fragments in registers at once than one loop over both):
 //   a1 = x[tok] @ W_in[g]      (gate and up, the forward's pre-activations, recomputed
 //                               in fp32 registers instead of being saved and re-read)
 //   G  = dout[tok] @ W_out[g]^T
@@ -332,7 +363,7 @@ combine_kernel(const typename Elem<DT>::T* __restrict__ rows, const int32_t* __r
 // Phase 3: dX rows = dA1 @ W_in[g]^T (W_in's rows are contiguous along 2H, the
 // contraction index), in passes of NP2 columns; reduced per token by `combine`.
 template <int DT, int NBW, int MR>
-__global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(ExpParams p) {
+__global__ void __launch_bounds__(NT, DT == DT_F32 ? 3 : 1) expert_bwd_kernel(ExpParams p) {
   using G = Geo<DT>;
   using T = typename G::T;
   using M = Mma<DT>;
@@ -342,8 +373,7 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
   constexpr int SA = RT * G::ROWB;
   constexpr int DA_PITCH = 2 * HPMAX * G::ES + 16;
   constexpr int Y_PITCH = NP2 * G::ES + 16;
-  __shared__ __attribute__((aligned(16))) char s_ax[2][SA];
-  __shared__ __attribute__((aligned(16))) char s_ad[2][SA];
+  __shared__ __attribute__((aligned(16))) char s_a[2][SA];
   __shared__ __attribute__((aligned(16))) char s_da[RT * DA_PITCH];
   // 32-bit rows go out from the accumulators (64-byte segments of a row)
   __shared__ __attribute__((aligned(16))) char s_y[DT == DT_F32 ? 16 : RT * Y_PITCH];
@@ -392,65 +422,30 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
   auto rowWo = [&](int n) -> const T* { return n < H ? Wout + (int64_t)n * d : nullptr; };
 
   // ---- phase 1: a1 = x W_in, G = dout W_out^T ----
-  DirectStage<DT, RT, NT> stX, stD;
+  constexpr bool ONE = DT == DT_F32;  // one buffer of weight fragments (k_loop)
   f32x4 acc1[MR][2 * NBW], accG[MR][NBW];  // a1 (gate blocks, then up blocks) and G
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
     for (int j = 0; j < NBW; ++j)
       acc1[i][j] = acc1[i][NBW + j] = accG[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Frag b0[3 * NBW], b1[3 * NBW];
-  auto loadB = [&](Frag* b, int kb) {
+  auto loadIn = [&](Frag* b, int kb) {
 #pragma unroll
     for (int j = 0; j < NBW; ++j) {
-      const int jb = wave * NBW + j;
-      b[j] = frag_pk<DT>(P1, jb, kb, p.in_kb);
-      b[NBW + j] = frag_pk<DT>(P1, HPMAX / 16 + jb, kb, p.in_kb);
-      if constexpr (DT == DT_F32)
-        b[2 * NBW + j] = frag_rows_quads(rowWo, jb * 16, kb * G::KC, d, fast);
-      else b[2 * NBW + j] = frag_rows<DT>(rowWo, jb * 16, kb * G::KC, d, fast);
+      b[j] = frag_pk<DT>(P1, wave * NBW + j, kb, p.in_kb);
+      b[NBW + j] = frag_pk<DT>(P1, HPMAX / 16 + wave * NBW + j, kb, p.in_kb);
     }
   };
-  const int nk = p.in_kb;
-  auto step = [&](int kc, const Frag* use, Frag* nxt) {
-    const bool more = kc + 1 < nk;
-    if (more) {
-      stX.load(rowX, (kc + 1) * G::KC, d, fast);
-      stD.load(rowD, (kc + 1) * G::KC, d, fast);
-      loadB(nxt, kc + 1);
-    }
-    Frag ax[MR], ad[MR];
+  auto loadOut = [&](Frag* b, int kb) {
 #pragma unroll
-    for (int i = 0; i < MR; ++i) {
-      ax[i] = frag_sw<DT>(s_ax[kc & 1], i * 16);
-      if constexpr (DT == DT_F32) ad[i] = frag_sw_halves(s_ad[kc & 1], i * 16);
-      else ad[i] = frag_sw<DT>(s_ad[kc & 1], i * 16);
+    for (int j = 0; j < NBW; ++j) {
+      const int n0 = (wave * NBW + j) * 16;
+      if constexpr (DT == DT_F32) b[j] = frag_rows_quads(rowWo, n0, kb * G::KC, d, fast);
+      else b[j] = frag_rows<DT>(rowWo, n0, kb * G::KC, d, fast);
     }
-    mma_tile<DT>(acc1, ax, use, rb);
-    if constexpr (DT == DT_F32) {
-      Frag wo[NBW];
-#pragma unroll
-      for (int j = 0; j < NBW; ++j) wo[j] = frag_from_quads(use[2 * NBW + j]);
-      mma_tile<DT>(accG, ad, wo, rb);
-    } else {
-      mma_tile<DT>(accG, ad, use + 2 * NBW, rb);
-    }
-    if (more) {
-      stX.store(s_ax[(kc + 1) & 1]);
-      stD.store(s_ad[(kc + 1) & 1]);
-    }
-    __syncthreads();
   };
-  stX.load(rowX, 0, d, fast);
-  stD.load(rowD, 0, d, fast);
-  loadB(b0, 0);
-  stX.store(s_ax[0]);
-  stD.store(s_ad[0]);
-  __syncthreads();
-  for (int kc = 0; kc < nk; kc += 2) {
-    step(kc, b0, b1);
-    if (kc + 1 < nk) step(kc + 1, b1, b0);
-  }
+  k_loop<DT, MR, 2 * NBW, false>(s_a, rowX, loadIn, p.in_kb, d, fast, acc1, rb);
+  k_loop<DT, MR, NBW, DT == DT_F32>(s_a, rowD, loadOut, p.in_kb, d, fast, accG, rb);
 
   // ---- phase 2: GLU backward, lane-local ----
   const T* bin = (g < p.E ? p.b_in : p.b_sh_in)
@@ -545,9 +540,9 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
     Frag c0[3], c1[3];
     loadB3(c0, 0);
     for (int q = 0; q < nk3; ++q) {
-      Frag* use = (q & 1) ? c1 : c0;
-      Frag* nxt = (q & 1) ? c0 : c1;
-      if (q + 1 < nk3) loadB3(nxt, q + 1);
+      Frag* use = !ONE && (q & 1) ? c1 : c0;
+      Frag* nxt = ONE || (q & 1) ? c0 : c1;
+      if (!ONE && q + 1 < nk3) loadB3(nxt, q + 1);
       const int half = q / nkh, kk = (q % nkh) * G::KC;
       const int kbyte = (half * HPMAX + kk) * G::ES;
       Frag af[MR];
@@ -560,6 +555,7 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 2 : 1) expert_bwd_kernel(Ex
         Frag wi[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) wi[j] = frag_from_quads(use[j]);
+        if (q + 1 < nk3) loadB3(nxt, q + 1);
         mma_tile<DT>(acc, af, wi, rb);
       } else {
         mma_tile<DT>(acc, af, use, rb);
@@ -961,9 +957,9 @@ static ExpParams make_params(const nsmoe_experts_args* a) {
 
 // 16-row blocks of a tile of the kernels of this file: 2 for fp32.  Its MFMAs run at a
 // sixteenth of the 16-bit rate, so a tile's time is its matrix work and small tiles cost
-// little in weight traffic; 32 rows take 26 to 50 KB of LDS, two workgroups per CU, where
+// little in weight traffic; 32 rows take 26 to 43 KB of LDS, three workgroups per CU, where
 // 64 took 100 KB and one, and share the work out in finer pieces (T = 2048: 550 tiles over
-// 256 CUs instead of 290).  expert_fwd 187 -> 140 us, expert_bwd 327 -> 257 us there.
+// 256 CUs instead of 290).  expert_fwd 187 -> 115 us, expert_bwd 327 -> 203 us there.
 static constexpr int gen_row_blocks(int dt) { return dt == DT_F32 ? 2 : 4; }
 
 static int64_t fwd_grid(const nsmoe_experts_args* a) {
