@@ -38,6 +38,7 @@ from torch import nn
 from . import _native as nat
 from .head import linear_cross_entropy
 from .moe import MoEBlock
+from .moe_kernel import _stream
 
 
 @dataclass
@@ -124,16 +125,23 @@ class Rotary:
 _ATTN_DT = {torch.bfloat16: nat.BF16, torch.float16: nat.F16}
 
 
+def _as(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """t in dtype and contiguous: t itself when it already is (a kernel's operand, read
+    through its pointer)."""
+    if t.dtype is dtype and t.is_contiguous():
+        return t
+    return t.detach().to(dtype).contiguous()
+
+
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """F.rms_norm(x, (d,), w, eps) of a contiguous 16-bit GPU tensor on the library's kernel
     (nsmoe_rms_norm).  Forward only."""
     d = x.shape[-1]
     y = torch.empty_like(x)
-    wc = w.detach().contiguous()
+    wc = _as(w, w.dtype)
     nat.check(nat.lib().nsmoe_rms_norm(_ATTN_DT[x.dtype], x.data_ptr(), wc.data_ptr(),
                                        float(eps), x.numel() // d, d, y.data_ptr(), None,
-                                       torch.cuda.current_stream().cuda_stream),
-              "nsmoe_rms_norm")
+                                       _stream()), "nsmoe_rms_norm")
     return y
 
 
@@ -153,17 +161,15 @@ def attn_prefill(qkv: torch.Tensor, B: int, T: int, n_heads: int, n_kv_heads: in
     dt = qkv.dtype
     qkv = qkv.contiguous()
     out = torch.empty((B * T, n_heads * 64), dtype=dt, device=qkv.device)
-    qg = q_gamma.detach().to(dt).contiguous()
-    kg = k_gamma.detach().to(dt).contiguous()
-    cos, sin = cos.float().contiguous(), sin.float().contiguous()
+    qg, kg = _as(q_gamma, dt), _as(k_gamma, dt)
+    cos, sin = _as(cos, torch.float32), _as(sin, torch.float32)
     a = nat.AttnArgs(dtype=_ATTN_DT[dt], n_heads=n_heads, n_kv_heads=n_kv_heads,
                      head_dim=64, batch=B, seq_len=T, ld=qkv.shape[1],
                      window=0 if window is None else int(window), eps=float(eps),
                      reserved=0, qkv=qkv.data_ptr(), q_gamma=qg.data_ptr(),
                      k_gamma=kg.data_ptr(), cos=cos.data_ptr(), sin=sin.data_ptr(),
                      out=out.data_ptr())
-    nat.check(nat.lib().nsmoe_attn_prefill(a, torch.cuda.current_stream().cuda_stream),
-              "nsmoe_attn_prefill")
+    nat.check(nat.lib().nsmoe_attn_prefill(a, _stream()), "nsmoe_attn_prefill")
     return out
 
 

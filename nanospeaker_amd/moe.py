@@ -201,6 +201,16 @@ class MoEBlock(nn.Module):
 
     # ---- forward -------------------------------------------------------------------------
 
+    def _set_results(self, counts, topk_idx, logits, aux) -> None:
+        """The side effects of a kernel-path call: plain attributes, set without
+        nn.Module.__setattr__'s search of parameters, buffers and modules (four searches
+        are a twentieth of a one-token call's host time)."""
+        put = object.__setattr__
+        put(self, "expert_counts", counts.detach())
+        put(self, "_routing", topk_idx)  # the last call's expert ids and router logits,
+        put(self, "_logits", logits)     # for inspection
+        put(self, "aux_loss", aux)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.shape[-1] != self.d_model:
             raise ValueError(f"expected last dim {self.d_model}, got {tuple(x.shape)}.")
@@ -217,10 +227,7 @@ class MoEBlock(nn.Module):
                 self.b_in, self.b_out, self.b_sh_in, self.b_sh_out, self.top_k,
                 self.router.wants_probs(), self.router.normalize_weights, self._kernel_act,
                 self.router.aux_loss_coef)
-            self.expert_counts = counts.detach()
-            self._routing = topk_idx  # the last call's expert ids and router logits,
-            self._logits = logits     # for inspection
-            self.aux_loss = aux
+            self._set_results(counts, topk_idx, logits, aux)
             return out.view(shape)
 
         topk_w, topk_idx, probs = self.router(x)
@@ -271,10 +278,7 @@ class MoEBlock(nn.Module):
                 self.b_in, self.b_out, self.b_sh_in, self.b_sh_out, self.top_k,
                 self.router.wants_probs(), self.router.normalize_weights, self._kernel_act,
                 self.router.aux_loss_coef, norm_w=gamma, norm_eps=float(eps))
-            self.expert_counts = counts.detach()
-            self._routing = topk_idx
-            self._logits = logits
-            self.aux_loss = aux
+            self._set_results(counts, topk_idx, logits, aux)
             return out.view(shape)
         return x + self(norm(x))
 

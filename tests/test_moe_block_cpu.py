@@ -225,3 +225,28 @@ def test_balance_loss_is_the_references():
     probs = torch.rand(16, 4).softmax(-1)
     counts = torch.tensor([5, 3, 8, 0])
     assert torch.equal(r.balance_loss(probs, counts), R.balance_loss(probs, counts, 1e-2, 4))
+
+
+def test_the_autograd_node_is_skipped_only_for_plain_inference():
+    """An eager kernel-path call runs its forward without the autograd node when nothing can
+    ask for a derivative: gradients on, a torch.func transform, a forward-mode level or a jit
+    trace keep the node (which differentiates, or raises for what it does not support)."""
+    import torch.autograd.forward_ad as fwAD
+
+    from nanospeaker_amd import moe_kernel as mk
+
+    assert not mk._plain_inference()
+    with torch.no_grad():
+        assert mk._plain_inference()
+        with torch.enable_grad():
+            assert not mk._plain_inference()
+        with fwAD.dual_level():
+            assert not mk._plain_inference()
+        seen = []
+        torch.func.vmap(lambda t: seen.append(mk._plain_inference()) or t)(torch.ones(2))
+        torch.jit.trace(lambda t: seen.append(mk._plain_inference()) or t + 1, torch.ones(2),
+                        check_trace=False)
+        assert seen == [False, False]
+        assert mk._plain_inference()
+    with torch.inference_mode():
+        assert mk._plain_inference()
