@@ -85,12 +85,22 @@ __device__ __forceinline__ int row16_sum_i(int v) {
   return v;
 }
 
-__device__ __forceinline__ int row16_min_i(int v) {
-  v = min(v, dpp_i<0xB1>(v));
-  v = min(v, dpp_i<0x4E>(v));
-  v = min(v, dpp_i<0x141>(v));
-  v = min(v, dpp_i<0x140>(v));
+__device__ __forceinline__ uint32_t row16_max_u(uint32_t v) {
+  v = max(v, (uint32_t)dpp_i<0xB1>((int)v));
+  v = max(v, (uint32_t)dpp_i<0x4E>((int)v));
+  v = max(v, (uint32_t)dpp_i<0x141>((int)v));
+  v = max(v, (uint32_t)dpp_i<0x140>((int)v));
   return v;
+}
+
+// A 16-bit value (held in fp32) as an order-preserving 16-bit integer; -0 maps to +0's image.
+// Every finite value and infinity maps above 0.
+template <int DT>
+__device__ __forceinline__ uint32_t ord16(float f) {
+  const auto v = Elem<DT>::from_f(f + 0.0f);  // -0 + 0 = +0
+  uint16_t b;
+  __builtin_memcpy(&b, &v, 2);
+  return (b & 0x8000u) ? (uint16_t)~b : (uint32_t)b | 0x8000u;
 }
 
 __device__ __forceinline__ float fmax_(float a, float b) { return fmaxf(a, b); }
@@ -354,12 +364,12 @@ __global__ void __launch_bounds__(W * 64, RtShape<W>::PER_CU) router_fwd_kernel(
     const int tl = wave * 4 + g;
     const int64_t t = tok0 + tl;
     const bool live = t < T;
-    float key[NB];
+    float key[NB], lg[NB];
     bool nan_here = false;
     float m = -INFINITY;
   #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      key[nb] = s_lg[tl * LGP + 16 * nb + j];
+      key[nb] = lg[nb] = s_lg[tl * LGP + 16 * nb + j];
       nan_here |= __builtin_isnan(key[nb]);
       m = fmaxf(m, key[nb]);
     }
@@ -382,7 +392,6 @@ __global__ void __launch_bounds__(W * 64, RtShape<W>::PER_CU) router_fwd_kernel(
           if (e < E) {
             const float p = ex[nb] * inv;
             if (live) a.probs[t * E + e] = p;
-            key[nb] = p;
             s_lg[tl * LGP + e] = p;  // the exact pass's keys and the column sums
           }
         }
@@ -392,33 +401,31 @@ __global__ void __launch_bounds__(W * 64, RtShape<W>::PER_CU) router_fwd_kernel(
       s_m[tl] = m;
       s_inv[tl] = inv;
     }
-    uint32_t avail = 0;
+    // k + 1 rounds of arg-max over (logit, lowest id) packed into one word: the 16-bit
+    // logit as an order-preserving integer above the id's complement, so a round is one
+    // maximum over the row's 16 lanes and its winner is unique.  (The keys of the train
+    // branch, the probabilities, fall with the logits.)  Lane j ends with rank j's word.
+    uint32_t pk[NB], c = 0xFFFFFFFFu, word = 0;
   #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) avail |= (16 * nb + j < E ? 1u : 0u) << nb;
-    bool exact = nan_row;
-    float s_sel = 0.0f;
-    int d_sel = 0;
-    for (int r = 0; r < k; ++r) {
-      float c = -INFINITY;
+    for (int nb = 0; nb < NB; ++nb)
+      pk[nb] = 16 * nb + j < E ? (ord16<DT>(lg[nb]) << 16) | (0xFFFFu - (16 * nb + j)) : 0u;
+    for (int r = 0; r <= k; ++r) {
+      uint32_t best = 0;
   #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-        if (avail >> nb & 1u) c = fmaxf(c, key[nb]);
-      const float mx = row16(c, fmax_);
-      int cnt = 0, loc = 1 << 20;
-  #pragma unroll
-      for (int nb = NB - 1; nb >= 0; --nb)
-        if ((avail >> nb & 1u) && key[nb] == mx) {
-          ++cnt;
-          loc = 16 * nb + j;
-        }
-      exact |= row16_sum_i(cnt) != 1;
-      const int id = row16_min_i(loc);
-      if ((id & 15) == j && id < (1 << 20)) avail &= ~(1u << (id >> 4));
-      if (j == r) {
-        s_sel = mx;
-        d_sel = id;
-      }
+      for (int nb = 0; nb < NB; ++nb) best = max(best, pk[nb] < c ? pk[nb] : 0u);
+      c = row16_max_u(best);  // 0: no expert left (k = E)
+      if (j == r) word = c;
     }
+    const int d_sel = 0xFFFF - (int)(word & 0xFFFFu);
+    const float s_sel = j < k ? s_lg[tl * LGP + d_sel] : 0.0f;
+    // The next rank's key: lane j + 1's, and for the last rank the round past it.  Ranks
+    // whose keys are not strictly falling go to the exact pass: equal keys, NaNs, and in
+    // the train branch probabilities within 8 ulp, where expf need not be monotone.
+    const uint32_t up = (uint32_t)dpp_i<0x101>((int)word);  // row_shl:1, on all lanes
+    const uint32_t nw = j == k - 1 ? c : up;
+    const float s_next = j < k && nw ? s_lg[tl * LGP + (0xFFFF - (int)(nw & 0xFFFFu))] : -INFINITY;
+    const bool falls = !(j < k && nw) || (train ? s_sel > s_next * 1.00000096f : s_sel > s_next);
+    const bool exact = nan_row || ((__ballot(!falls) >> (16 * g)) & 0xFFFFull) != 0;
     {
       const bool o = j < k;
       const float s = o ? s_sel : 0.0f;

@@ -79,6 +79,12 @@ struct RegRow {
     k1 = put_lane(k1, kb, l1, lane);
     i1 = put_lane(i1, v.id, l1, lane);
   }
+  // The same for i < 64.
+  __device__ __forceinline__ KV get_lo(int i) const { return KV{(uint32_t)rl(k0, i), rl(i0, i)}; }
+  __device__ __forceinline__ void set_lo(int i, KV v) {
+    k0 = put_lane(k0, (int)v.key, i, lane);
+    i0 = put_lane(i0, v.id, i, lane);
+  }
   __device__ __forceinline__ void swap(int i, int j) {
     const KV t = get(i);
     set(i, get(j));
@@ -338,6 +344,41 @@ __device__ __forceinline__ int partition_parallel(RegRow& a, int first, int last
   return lnext < rprev ? lnext : rprev;
 }
 
+// The same partition for a range inside the first 64 positions (0 <= first, last <= 64), where
+// one register pair holds it: half the compares, masks and LDS traffic.  After the first
+// rounds the range is almost always there (top-6 of 76).
+__device__ __forceinline__ int partition_parallel_lo(RegRow& a, int first, int last, int2* kv,
+                                                     uint32_t pk) {
+  const uint32_t x = (uint32_t)a.k0;
+  const uint64_t below = ~0ull >> (64 - last);
+  const uint64_t bl = __builtin_amdgcn_ballot_w64(x <= pk) & below & (~0ull << (first + 1));
+  const uint64_t br = __builtin_amdgcn_ballot_w64(x >= pk) & below & (~0ull << first);
+  const bool isL = (bl >> a.lane) & 1ull, isR = (br >> a.lane) & 1ull;
+  const int rl = mbcnt64(bl);
+  const int ar = __builtin_popcountll(br) - mbcnt64(br) - (isR ? 1 : 0);
+  const int istar = __builtin_popcountll(bl & __builtin_amdgcn_ballot_w64(ar > rl));
+  if (istar == 0) return bl ? ff1_64(bl) : 63;
+  const bool sl = isL && rl < istar, sr = isR && ar < istar;  // disjoint positions
+  if (sl || sr) kv[sl ? rl : 64 + ar] = make_int2(a.k0, a.i0);
+  const uint64_t nl = bl & __builtin_amdgcn_ballot_w64(rl == istar);
+  const uint64_t mr = br & __builtin_amdgcn_ballot_w64(ar == istar - 1);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (sl || sr) {
+    const int2 v = kv[sl ? 64 + rl : ar];
+    a.k0 = v.x;
+    a.i0 = v.y;
+  }
+  // the next round's writes to kv must not overtake these reads
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int lnext = nl ? ff1_64(nl) : 1 << 20;
+  const int rprev = mr ? ff1_64(mr) : 63;
+  return lnext < rprev ? lnext : rprev;
+}
+
 // libstdc++'s insertion sort with a strict comparator moves an element left only past
 // elements it ranks strictly before, so it is the stable sort: the element at p lands at
 // first + #{q : a[q] before a[p]} + #{q < p : a[q] equivalent to a[p]}.  For ranges
@@ -377,7 +418,10 @@ __device__ __forceinline__ void nth_element_par(RegRow& a, int nth, int n, int2*
     // move_median_to_first(first, first + 1, mid, last - 1) from one read of the four
     // positions: the swap's values are then known scalars, and so is the pivot's key.
     const int x = first + 1, y = first + (last - first) / 2, z = last - 1;
-    const KV ef = a.get(first), ex = a.get(x), ey = a.get(y), ez = a.get(z);
+    const bool lo = last <= 64;  // uniform: the range lies in the first register pair
+    KV ef, ex, ey, ez;
+    if (lo) ef = a.get_lo(first), ex = a.get_lo(x), ey = a.get_lo(y), ez = a.get_lo(z);
+    else ef = a.get(first), ex = a.get(x), ey = a.get(y), ez = a.get(z);
     int m;
     KV em;
     if (gt(ex, ey)) {
@@ -391,9 +435,16 @@ __device__ __forceinline__ void nth_element_par(RegRow& a, int nth, int n, int2*
     } else {
       m = y, em = ey;
     }
-    a.set(first, em);
-    a.set(m, ef);
-    const int cut = partition_parallel(a, first, last, pos, em.key);
+    int cut;
+    if (lo) {
+      a.set_lo(first, em);
+      a.set_lo(m, ef);
+      cut = partition_parallel_lo(a, first, last, pos, em.key);
+    } else {
+      a.set(first, em);
+      a.set(m, ef);
+      cut = partition_parallel(a, first, last, pos, em.key);
+    }
     if (cut <= nth) first = cut;
     else last = cut;
   }

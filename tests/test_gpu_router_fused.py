@@ -14,7 +14,7 @@ import pytest
 import torch
 
 from oracle import moe_ref as R
-from tests.helpers import assert_close_bf16
+from tests.helpers import assert_close_bf16, lib_options
 
 pytestmark = pytest.mark.gpu
 
@@ -32,6 +32,8 @@ def run(T, E, k, train, normalize, dtype=torch.bfloat16, d=64, mode="rand", bias
     x = torch.randn(T, d, generator=g).to(dtype)
     if mode == "zeros":
         x[::3] = 0
+    if mode == "allzero":
+        x[:] = 0
     if mode == "nan":
         x[::5, 3] = float("nan")
     H = 32
@@ -89,6 +91,41 @@ def test_fused_router_shapes(T, E, k):
     run(T, E, k, True, True, mode="pairs" if T % 2 else "rand", seed=T + E)
 
 
+def _special_logits(kind):
+    """[80] logits that sit on the fast selection's edges."""
+    v = torch.linspace(-3, 3, 80)[torch.randperm(80, generator=torch.Generator().manual_seed(5))]
+    top = v.argsort(descending=True)
+    if kind == "tie past the last rank":      # ranks k - 1 and k only
+        v[top[6]] = v[top[5]]
+    elif kind == "tie inside":                # ranks 2 and 3 only
+        v[top[3]] = v[top[2]]
+    elif kind == "tie below":                 # ranks k and k + 1: not selected, no exact pass
+        v[top[7]] = v[top[6]]
+    elif kind == "probabilities collapse":    # distinct logits, equal exp(l - max)
+        v = torch.arange(1, 81).float() * 1e-10
+    elif kind == "signed zeros":
+        v = -v.abs() - 1
+        v[[3, 40, 41, 66, 70, 71, 72]] = torch.tensor([0.0, -0.0, 0.0, -0.0, -0.0, 0.0, 1.0])
+    elif kind == "inf":
+        v[17] = float("inf")
+    elif kind == "mostly -inf":
+        v[torch.arange(80) % 16 != 3] = float("-inf")
+    return v
+
+
+@pytest.mark.parametrize("waves", [8, 16])
+@pytest.mark.parametrize("kind", ["tie past the last rank", "tie inside", "tie below",
+                                  "probabilities collapse", "signed zeros", "inf",
+                                  "mostly -inf"])
+def test_fused_router_selection_edges(kind, waves):
+    """The arg-max rounds against CPU topk where a row is just tied or just not, in both
+    branches: the logits come in as the offset on zero tokens."""
+    with lib_options(router_waves=waves):
+        for train in ((False,) if kind == "inf" else (True, False)):
+            run(37, 80, 6, train, True, mode="allzero", bias=_special_logits(kind))
+            run(5, 80, 16, train, True, mode="allzero", bias=_special_logits(kind))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fused_router_dtypes_and_width(dtype):
     run(777, 76, 6, True, True, dtype=dtype, d=576, seed=3)
@@ -114,7 +151,6 @@ def test_fused_router_both_workgroup_shapes(T, E, k, d, mode, dtype):
     two (the second partial), 160 and 64 one.  Each shape's routing is bit-exact against
     the oracle on its own logits, and the two shapes' logits are bit-identical (every
     logit is the same MFMA chain over the same k-steps in the same order)."""
-    from tests.helpers import lib_options
 
     got = {}
     for waves in (16, 8):
