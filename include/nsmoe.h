@@ -313,6 +313,11 @@ int nsmoe_experts_bwd(const nsmoe_experts_args* args, const int32_t* inv,
  *     d(logits) as nsmoe_route_bwd writes it, grad_w_router is unused; workspace
  *     nsmoe_block_bwd_workspace_size(args, route_flags, 0).
  *
+ * NSMOE_BLOCK_INFER in the forward's route_flags says that no backward follows: the
+ * dispatch's parts of `saved` (sorted ids, block owners, offsets, the padded total, inv)
+ * may then be left unwritten, as a decode-sized call does, whose expert kernel finds its
+ * rows in topk_idx without a dispatch.  Every other output is the same.
+ *
  * The RMSNorm and residual around the block (`norm` non-NULL, NSMOE_BLOCK_NORM in
  * route_flags; both or neither): the FFN half of the reference's Block.forward,
  *   out = x + MoEBlock(RMSNorm(x))          (src/model/nanospeaker.py:169, ln.py:30-36)
@@ -333,6 +338,7 @@ typedef struct nsmoe_block_norm {
 } nsmoe_block_norm;
 
 #define NSMOE_BLOCK_NORM 32
+#define NSMOE_BLOCK_INFER 64
 #define NSMOE_BLOCK_PACK 8
 #define NSMOE_BLOCK_SAVE_ACT 16
 

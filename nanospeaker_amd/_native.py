@@ -14,7 +14,7 @@ LIB_PATH = Path(__file__).resolve().parent / "libnsmoe.so"
 
 BF16, F16, F32 = 0, 1, 2
 ROUTE_PROBS, ROUTE_NORMALIZE, ROUTE_LOGITS16 = 1, 2, 4
-BLOCK_PACK, BLOCK_SAVE_ACT, BLOCK_NORM = 8, 16, 32
+BLOCK_PACK, BLOCK_SAVE_ACT, BLOCK_NORM, BLOCK_INFER = 8, 16, 32, 64
 ABI_VERSION = 8
 
 # Every symbol include/nsmoe.h declares, with (restype, argtypes).

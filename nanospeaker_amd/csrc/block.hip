@@ -217,6 +217,13 @@ extern "C" int nsmoe_block_fwd(const nsmoe_experts_args* a, const nsmoe_block_no
       r.xn = sv + L.off[NSMOE_SAVED_XN];
       r.rstd = (float*)(sv + L.off[NSMOE_SAVED_RSTD]);
     }
+    // A decode-sized forward that no backward follows needs no dispatch: its expert tiles
+    // find their rows in the expert ids themselves.
+    if ((route_flags & NSMOE_BLOCK_INFER) && !probs && !pack && experts_scan_supported(&b)) {
+      NSMOE_TRY(router_fused_launch(r, a->dtype, s));
+      return experts_fwd_scan_launch(&b, topk_idx, counts, (uint32_t*)aux, out, ws + dsp, exp, s,
+                                     norm ? a->x : nullptr);
+    }
     if (rc == NSMOE_OK) rc = router_fused_launch(r, a->dtype, s);
     BalanceArgs fold{r.colsum, router_fused_chunks(T), T, aux_coef, aux};
     if (rc == NSMOE_OK)

@@ -233,7 +233,8 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 3 : 1) expert_fwd_kernel(Ex
 // out[t] = sum_j rows[inv[t * k + j]] + sum_s rows[l_cap + s * T + t], fp32 accumulation
 // in the order routed j = 0 .. k - 1, then shared s = 0 .. S - 1.  With `resid` the sum,
 // rounded to the dtype, is added to resid[t] and rounded again: the block output plus the
-// residual stream, as `x + ffn(norm(x))` computes it (nanospeaker.py:169).
+// residual stream, as `x + ffn(norm(x))` computes it (nanospeaker.py:169).  Without inv the
+// row of pair t k + j is row t k + j.
 constexpr int COMBINE_KMAX = 8;  // top_k and shared-expert counts of the gather fast path
 constexpr int COMBINE_SMAX = 2;
 template <int DT>
@@ -265,7 +266,8 @@ combine_kernel(const typename Elem<DT>::T* __restrict__ rows, const int32_t* __r
       const int c = (i - t * vpr) * G::VE;
       int32_t sl[COMBINE_KMAX];
 #pragma unroll
-      for (int j = 0; j < COMBINE_KMAX; ++j) sl[j] = j < k ? inv[(int64_t)t * k + j] : -1;
+      for (int j = 0; j < COMBINE_KMAX; ++j)
+        sl[j] = j < k ? (inv ? inv[(int64_t)t * k + j] : t * k + j) : -1;
       u32x4 v[COMBINE_KMAX + COMBINE_SMAX];
 #pragma unroll
       for (int j = 0; j < COMBINE_KMAX; ++j) {
@@ -304,7 +306,7 @@ combine_kernel(const typename Elem<DT>::T* __restrict__ rows, const int32_t* __r
 #pragma unroll
       for (int e = 0; e < G::VE; ++e) acc[e] = 0.0f;
       for (int j = 0; j < k; ++j) {
-        const int32_t s = inv[t * k + j];
+        const int32_t s = inv ? inv[t * k + j] : (int32_t)(t * k + j);
         if (s < 0) continue;
         u32x4 v = *(const u32x4*)(rows + (int64_t)s * d + c);
         TT tmp[G::VE];
@@ -333,7 +335,7 @@ combine_kernel(const typename Elem<DT>::T* __restrict__ rows, const int32_t* __r
       const int c = (int)(i % d);
       float acc = 0.0f;
       for (int j = 0; j < k; ++j) {
-        const int32_t s = inv[t * k + j];
+        const int32_t s = inv ? inv[t * k + j] : (int32_t)(t * k + j);
         if (s >= 0) acc += Elem<DT>::to_f(rows[(int64_t)s * d + c]);
       }
       for (int s = 0; s < S; ++s)
@@ -1041,6 +1043,23 @@ static int experts_fwd_impl(const nsmoe_experts_args* a, const int32_t* inv, voi
                             out, fast, s, resid);
 }
 
+// The decode-sized forward without a dispatch (experts_fwd_scan_launch).
+template <int DT>
+static int experts_scan_impl(const nsmoe_experts_args* a, const int64_t* topk_idx,
+                             int32_t* counts, uint32_t* zero4, void* out, void* ws,
+                             const void* resid, hipStream_t s) {
+  ExpParams p = make_params(a);
+  p.y = ws;
+  p.topk_idx = topk_idx;
+  p.counts_out = counts;
+  p.zero4 = zero4;
+  const int rc = launch_fwd_async(DT, p, nbw_for(a), 1, s);
+  NSMOE_REQUIRE(rc != -1, "experts_fwd_scan: unsupported shape");
+  NSMOE_TRY(rc);
+  return launch_combine<DT>(ws, nullptr, a->n_tokens, a->d_model, a->top_k, a->n_shared, a->l_cap,
+                            out, p.fast && aligned16(out) && aligned16(resid), s, resid);
+}
+
 struct BwdLayout {
   size_t da1, hbuf, dxrow, p_in, p_out, total;
 };
@@ -1227,6 +1246,31 @@ int experts_fwd_launch(const nsmoe_experts_args* a, const int32_t* inv, void* ou
     case DT_F16: return experts_fwd_impl<DT_F16>(a, inv, out, workspace, act_out, resid, s);
     default: return experts_fwd_impl<DT_F32>(a, inv, out, workspace, act_out, resid, s);
   }
+}
+
+bool experts_scan_supported(const nsmoe_experts_args* a) {
+  return a->n_tokens > 0 && a->dtype != DT_F32 &&
+         fwd_scan_shape(a->dtype, make_params(a), nbw_for(a));
+}
+
+int experts_fwd_scan_launch(const nsmoe_experts_args* a, const int64_t* topk_idx, int32_t* counts,
+                            uint32_t* zero4, void* out, void* workspace, size_t workspace_bytes,
+                            hipStream_t s, const void* resid) {
+  NSMOE_TRY(validate(a));
+  NSMOE_REQUIRE(a->x && a->topk_w && topk_idx && counts && out && a->w_in_packed &&
+                    a->w_out_packed, "experts_fwd_scan: NULL pointer");
+  if (!experts_scan_supported(a)) {
+    set_error("experts_fwd_scan: unsupported shape");
+    return NSMOE_EINVAL;
+  }
+  const size_t need = nsmoe_experts_fwd_workspace_size(a);
+  if (workspace_bytes < need || !workspace) {
+    set_error("experts_fwd_scan: workspace %zu B < %zu B", workspace_bytes, need);
+    return NSMOE_EWORKSPACE;
+  }
+  return a->dtype == DT_BF16
+             ? experts_scan_impl<DT_BF16>(a, topk_idx, counts, zero4, out, workspace, resid, s)
+             : experts_scan_impl<DT_F16>(a, topk_idx, counts, zero4, out, workspace, resid, s);
 }
 
 }  // namespace nsmoe

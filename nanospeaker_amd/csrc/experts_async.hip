@@ -34,7 +34,8 @@ namespace nsmoe {
 template <int DT>
 __device__ __forceinline__ void store_block48(const uint32_t (&lo)[3], const uint32_t (&hi)[3],
                                               typename Elem<DT>::T* Y, int d, int row0,
-                                              int rows, int cw, int lane) {
+                                              int rows, int cw, int lane,
+                                              const int* slot = nullptr) {
   using T = typename Elem<DT>::T;
   if (cw + 32 <= d) {
     const auto l32 = __builtin_amdgcn_permlane32_swap(lo[0], lo[1], false, false);
@@ -46,13 +47,15 @@ __device__ __forceinline__ void store_block48(const uint32_t (&lo)[3], const uin
     const uint32_t b2lo = bperm(qa, lo[2]), b2hi = bperm(qa, hi[2]);
     const int m = row0 + (lane >> 2), c = lane & 3;
     if (m < rows) {
-      T* yrow = Y + (int64_t)m * d;
+      T* yrow = Y + (int64_t)(slot ? slot[m] : m) * d;
       *(u32x4*)(yrow + cw + c * 8) = v;
       if (cw + 32 < d) *(uint2*)(yrow + cw + 32 + c * 4) = make_uint2(b2lo, b2hi);
     }
   } else if (cw < d) {
     const int m = row0 + (lane & 15);
-    if (m < rows) *(uint2*)(Y + (int64_t)m * d + cw + (lane >> 4) * 4) = make_uint2(lo[0], hi[0]);
+    if (m < rows)
+      *(uint2*)(Y + (int64_t)(slot ? slot[m] : m) * d + cw + (lane >> 4) * 4) =
+          make_uint2(lo[0], hi[0]);
   }
 }
 
@@ -296,7 +299,14 @@ __global__ void __launch_bounds__(NT, 2) expert_fwd_async_kernel(ExpParams p) {
 // unconditional (out-of-range fragments read a zero page), so the compiler's own waits
 // for the weight registers are exact or stricter and leave the next step's loads in flight.
 // Shapes: d % 64 == 0 (an even number of GEMM1 steps) and an even number of GEMM2 steps.
-template <int DT, int NBW, int MB, int D>
+//
+// SCAN (32-row tiles, at most SCAN_MAX_PAIRS pairs): there is no dispatch before this launch.
+// Tile `local` of group g is workgroup local (E + S) + g', shared groups first; its four
+// waves look for g in the routed expert ids (ballots keep the pairs' order) and take the
+// matches 32 local .. + 31 as the tile's rows, whose outputs go to row `pair` of y.  The
+// ids are a few KB from L2, so scanning them in every tile costs less than the place
+// launch (6.8 us at T = 64) and this kernel's own lookups of its result.
+template <int DT, int NBW, int MB, int D, bool SCAN = false>
 __global__ void __launch_bounds__(NT, MB > 2 && (MB == 6 || D == 3) ? 3 : 2)
 expert_fwd_reg_kernel(ExpParams p) {
   using G = Geo<DT>;
@@ -331,20 +341,70 @@ expert_fwd_reg_kernel(ExpParams p) {
   __shared__ __attribute__((aligned(16))) char s_h[TM * HP_PITCH];
   __shared__ int s_tok[TM];
   __shared__ float s_w[TM];
-  __shared__ int s_loc[3];
+  __shared__ int s_loc[SCAN ? 4 : 3];
+  __shared__ int s_slot[SCAN ? TM : 1];  // the rows' places in y
+  static_assert(!SCAN || MB == 2, "scanning tiles have 32 rows");
 
-  const int tile = tile_of_block(p);
-  Located loc;
-  if (!locate(tile, p.E + p.S, [&](int g) { return (rows_of(p, g) + TM - 1) / TM; },
-              [](int) { return 0; }, s_loc, loc))
-    return;
-  const int g = loc.g, m0 = loc.local * TM;
-  const int rows = min(TM, rows_of(p, g) - m0);
-  const int64_t slot0 = row_start(p, g) + m0;
+  int g, m0, rows;
+  int64_t slot0;
+  if constexpr (SCAN) {
+    const int v = blockIdx.x % (p.E + p.S), local = blockIdx.x / (p.E + p.S);
+    g = v < p.S ? p.E + v : v - p.S;
+    m0 = local * TM;
+    slot0 = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.zero4) *p.zero4 = 0u;
+    if (g >= p.E) {
+      rows = min(TM, (int)p.T - m0);
+      if ((int)threadIdx.x < rows)
+        s_slot[threadIdx.x] = (int)(p.l_cap + (int64_t)(g - p.E) * p.T) + m0 + threadIdx.x;
+    } else {
+      constexpr int R = SCAN_MAX_PAIRS / NT;  // ids a lane
+      const int M = (int)p.T * p.k, per = (M + NT - 1) / NT * 64;  // pairs a wave
+      const int p0 = (threadIdx.x >> 6) * per + (threadIdx.x & 63), p1 = p0 - (threadIdx.x & 63) + per;
+      int id[R], at[R], cnt = 0;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        id[r] = p0 + 64 * r < min(M, p1) ? (int)p.topk_idx[p0 + 64 * r] : -1;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const uint64_t hit = __ballot(id[r] == g);
+        at[r] = cnt + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hit >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)hit, 0u));
+        cnt += __popcll(hit);
+      }
+      if ((threadIdx.x & 63) == 0) s_loc[threadIdx.x >> 6] = cnt;
+      __syncthreads();
+      int base = 0, total = 0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        if (w < (int)(threadIdx.x >> 6)) base += s_loc[w];
+        total += s_loc[w];
+      }
+      if (local == 0 && threadIdx.x == 0) p.counts_out[g] = total;
+      rows = min(TM, total - m0);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int q = base + at[r] - m0;
+        if (id[r] == g && q >= 0 && q < TM) s_slot[q] = p0 + 64 * r;
+      }
+    }
+    if (rows <= 0) return;  // uniform
+    __syncthreads();
+  } else {
+    const int tile = tile_of_block(p);
+    Located loc;
+    if (!locate(tile, p.E + p.S, [&](int g) { return (rows_of(p, g) + TM - 1) / TM; },
+                [](int) { return 0; }, s_loc, loc))
+      return;
+    g = loc.g;
+    m0 = loc.local * TM;
+    rows = min(TM, rows_of(p, g) - m0);
+    slot0 = row_start(p, g) + m0;
+  }
   // The first saved pre-activation block of the tile, read here with the other group
   // offsets: inside the epilogue the load of offs[g] would come after the block stores
   // and the GEMM2 weight loads, and waiting for it would wait for all of them.
-  const int64_t a1_blk0 = p.a1_out ? act_block(p, g, m0) : 0;
+  const int64_t a1_blk0 = !SCAN && p.a1_out ? act_block(p, g, m0) : 0;
   const int tid = threadIdx.x, lane = tid & 63, lc = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d = p.d, H = p.H, twoH = 2 * p.H;
@@ -399,7 +459,7 @@ expert_fwd_reg_kernel(ExpParams p) {
     int tok = -1;
     if (tid < rows) {
       if (routed) {
-        pair = p.sorted_ids[slot0 + tid];
+        pair = SCAN ? s_slot[tid] : p.sorted_ids[slot0 + tid];
         tok = pair / p.k;
       } else {
         tok = m0 + tid;
@@ -645,7 +705,7 @@ expert_fwd_reg_kernel(ExpParams p) {
           // live through GEMM1 (the kernel is at its register cap).
           int sl = lane;
           asm volatile("" : "+v"(sl));
-          store_block48<DT>(lo, hi, Y, d, i * 16, rows, cw, sl);
+          store_block48<DT>(lo, hi, Y, d, i * 16, rows, cw, sl, SCAN ? s_slot : nullptr);
         }
       }
     }
@@ -2094,6 +2154,12 @@ static int64_t tile_grid(const ExpParams& p, int bm) {
 
 template <int DT, int NBW>
 static void fwd_reg_launch(const ExpParams& p, int mb, int dist, hipStream_t s) {
+  if (p.topk_idx) {  // fwd_scan_shape
+    const unsigned gs = (unsigned)((p.E + p.S) * cdiv(p.T, 32));
+    if (dist == 6) expert_fwd_reg_kernel<DT, NBW, 2, 6, true><<<gs, NT, 0, s>>>(p);
+    else expert_fwd_reg_kernel<DT, NBW, 2, 2, true><<<gs, NT, 0, s>>>(p);
+    return;
+  }
   if (mb == 2) {
     const unsigned g2 = (unsigned)tile_grid(p, 32);
     if (dist == 6) expert_fwd_reg_kernel<DT, NBW, 2, 6><<<g2, NT, 0, s>>>(p);
@@ -2110,20 +2176,34 @@ static void fwd_reg_launch(const ExpParams& p, int mb, int dist, hipStream_t s) 
   }
 }
 
+// Row blocks of the register-tiled forward's tiles: 96 rows once 64-row tiles overflow the
+// resident workgroup slots (3 per CU); 32 rows (at prefetch distance 6) while 64-row tiles
+// would fill under half the CUs (decode-sized calls: a tile's time is its weight stream's
+// latency, not its rows).  The "fwd_rows" option forces a tile height.
+static int fwd_row_blocks(const ExpParams& p) {
+  if (const int64_t v = option(OPT_FWD_ROWS)) return (int)(v / 16);
+  const int64_t g64 = tile_grid(p, 64);
+  return g64 > 3 * (int64_t)device_cus() ? 6 : 2 * g64 <= device_cus() ? 2 : 4;
+}
+
+// d and the step counts the register-tiled forward unrolls by.
+static bool fwd_reg_shape(const ExpParams& p) {
+  return p.d % 64 == 0 && (((p.d + NP2 - 1) / NP2) * p.out_kb) % 2 == 0;
+}
+
+bool fwd_scan_shape(int dtype, const ExpParams& p, int nbw) {
+  return p.fast && nbw <= 2 && (dtype == DT_BF16 || dtype == DT_F16) && fwd_reg_shape(p) &&
+         p.T * p.k <= SCAN_MAX_PAIRS && fwd_row_blocks(p) == 2;
+}
+
 int launch_fwd_async(int dtype, const ExpParams& p, int nbw, int64_t grid, hipStream_t s) {
   if (!p.fast || nbw > 2 || (dtype != DT_BF16 && dtype != DT_F16)) return -1;
   if (grid <= 0) return NSMOE_OK;
   constexpr int S = 3;
   KernelTimer timer("expert_fwd", s);
   const int n2 = ((p.d + NP2 - 1) / NP2) * p.out_kb;
-  if (p.d % 64 == 0 && n2 % 2 == 0) {
-    // 96-row tiles once 64-row tiles overflow the resident workgroup slots (3 per CU);
-    // 32-row tiles at prefetch distance 6 while 64-row tiles would fill under half the
-    // CUs (decode-sized calls: a tile's time is its weight stream's latency, not its
-    // rows).  The "fwd_rows" option forces a tile height.
-    const int64_t g64 = tile_grid(p, 64);
-    int mb = g64 > 3 * (int64_t)device_cus() ? 6 : 2 * g64 <= device_cus() ? 2 : 4;
-    if (const int64_t v = option(OPT_FWD_ROWS)) mb = (int)(v / 16);
+  if (fwd_reg_shape(p)) {
+    const int mb = fwd_row_blocks(p);
     // Prefetch distance 2 (6 for 32-row tiles); the "fwd_dist" option asks for another,
     // taken where both GEMMs' step counts are multiples of it (6: 32-row tiles only).
     const int nk1 = p.in_kb;

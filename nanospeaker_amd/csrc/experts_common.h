@@ -39,6 +39,11 @@ struct ExpParams {
   int in_kb, in_nb, out_kb, out_nb;
   // forward output rows
   void* y;
+  // Decode-sized forwards (expert_fwd_reg_kernel, SCAN): the routed expert ids [T, k] the
+  // tiles find their rows in, the routing counts they leave, and four bytes to clear.
+  const int64_t* topk_idx;
+  int32_t* counts_out;
+  uint32_t* zero4;
   // The pre-activations a1 = x W_in + b_in in 16 x 16 blocks (act_block): written by the
   // forward when a1_out is set, read by the backward (instead of being recomputed) when
   // a1_in is set.
@@ -154,6 +159,10 @@ __device__ __forceinline__ int dw_shared_partials(const ExpParams& p) {
 // Async (direct-to-LDS) variants for 16-bit types and d_hidden <= 128; each returns
 // NSMOE_OK after launching, or -1 when the shape is not one they take.
 int launch_fwd_async(int dtype, const ExpParams& p, int nbw, int64_t grid, hipStream_t s);
+// Whether launch_fwd_async takes p with 32-row tiles, and the call is small enough for its
+// tiles to scan the expert ids (p.topk_idx set).
+bool fwd_scan_shape(int dtype, const ExpParams& p, int nbw);
+constexpr int SCAN_MAX_PAIRS = 2048;  // 8 ids a lane
 // Both dW modes in one launch (q_in: dW_in, q_out: dW_out pointers and partials).
 int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_out,
                          int64_t routed_chunks, hipStream_t s);
@@ -196,4 +205,12 @@ int experts_fwd_launch(const ::nsmoe_experts_args* a, const int32_t* inv, void* 
 // that write and read them do not apply (16-bit types, d % 64 == 0, H % 16 == 0, H <= 128
 // and the step-count parities of the register-tiled forward and backward).
 size_t experts_save_act_bytes(const ::nsmoe_experts_args* a);
+// The same forward for a decode-sized call straight from the router's expert ids, with no
+// dispatch: the expert tiles find their rows in topk_idx [T, k] and write counts [E] (and
+// four zero bytes at zero4 when it is not NULL); a->sorted_ids, pad_offsets and counts are
+// not read.  Only where experts_scan_supported(a).
+int experts_fwd_scan_launch(const ::nsmoe_experts_args* a, const int64_t* topk_idx,
+                            int32_t* counts, uint32_t* zero4, void* out, void* workspace,
+                            size_t workspace_bytes, hipStream_t stream, const void* resid);
+bool experts_scan_supported(const ::nsmoe_experts_args* a);
 }  // namespace nsmoe

@@ -898,7 +898,7 @@ def norm_fusable(dtype: torch.dtype, d: int, e: int, k: int) -> bool:
 
 def _block_fwd_impl(x, W_r, w_in, w_out, w_sh_in, w_sh_out, b_in, b_out, b_sh_in, b_sh_out,
                     top_k, want_probs, normalize, activation, aux_coef, logit_bias=None,
-                    save_act=False, norm_w=None, norm_eps=1e-6):
+                    save_act=False, norm_w=None, norm_eps=1e-6, infer=False):
     """
     MoEBlock.forward's kernel path (moe.py:345-418): the router GEMM `x @ W_r` (torch,
     router.py:69), then one C call (nsmoe_block_fwd: router tail, dispatch, routed + shared
@@ -921,6 +921,9 @@ def _block_fwd_impl(x, W_r, w_in, w_out, w_sh_in, w_sh_out, b_in, b_out, b_sh_in
     With `norm_w` [d] (an RMSNorm gain; norm_fusable shapes) x is the residual stream and
     `out` is x + block(rms_norm(x, norm_w, norm_eps)) (nsmoe.h NSMOE_BLOCK_NORM): the
     Block's FFN half, nanospeaker.py:169.
+
+    With `infer` no backward follows: the dispatch's part of `saved` may be left unwritten
+    (nsmoe.h NSMOE_BLOCK_INFER).
     """
     dev, dt = x.device, x.dtype
     n, d = x.shape
@@ -966,7 +969,8 @@ def _block_fwd_impl(x, W_r, w_in, w_out, w_sh_in, w_sh_out, b_in, b_out, b_sh_in
             nrm.weight, nrm.grad_weight, nrm.eps = norm_w.data_ptr(), None, float(norm_eps)
         nat.check(nat.lib().nsmoe_block_fwd(
             a, nrm, W_r.data_ptr() if plan.fuse_route else None, _p(bias), logits.data_ptr(),
-            flags | (nat.BLOCK_PACK if pending is not None else 0), aux_coef,
+            flags | (nat.BLOCK_PACK if pending is not None else 0)
+            | (nat.BLOCK_INFER if infer else 0), aux_coef,
             saved.data_ptr(), topk_idx.data_ptr(), counts.data_ptr(), out.data_ptr(),
             aux_buf.data_ptr(), ws.data_ptr(), plan.fwd_ws, _stream()),
             "nsmoe_block_fwd")
@@ -1181,6 +1185,11 @@ class _BlockEager(torch.autograd.Function):
         return _block_backward(ctx, g_out, g_aux, _block_bwd_impl)
 
 
+def _block_fwd_infer(*inputs):
+    """_block_fwd_impl for a call that no backward follows."""
+    return _block_fwd_impl(*inputs, infer=True)
+
+
 def _plain_inference() -> bool:
     """Whether nothing can ask an eager call for a derivative or a transform: gradients off,
     no torch.func transform, no forward-mode level and no jit trace.  The autograd node
@@ -1228,7 +1237,7 @@ def block_forward_state(x, router_W, w_in, w_out, w_sh_in, w_sh_out, b_in, b_out
     if torch.compiler.is_compiling():
         op = block_fwd
     else:
-        op = _block_fwd_impl if _plain_inference() else _BlockEager.apply
+        op = _block_fwd_infer if _plain_inference() else _BlockEager.apply
     # The pre-activations are saved only for a forward that autograd will run backward
     # through (a checkpointed block's first, gradient-free forward does not save them).
     params = (router_W, w_in, w_out, w_sh_in, w_sh_out, b_in, b_out, b_sh_in, b_sh_out, norm_w)

@@ -264,6 +264,40 @@ def test_dw_chunk_edges(T, dtype):
     run_case(T, train=True, backward=True, d=128, E=8, d_ff=96, k=4, S=1, dtype=dtype)
 
 
+@pytest.mark.parametrize("collapsed", [False, True])
+@pytest.mark.parametrize("T", [1, 2, 31, 32, 33, 64, 65, 170, 341, 342])
+def test_decode_without_dispatch_matches_the_dispatched_forward(T, collapsed):
+    """Decode-sized calls without gradients find their rows in the expert ids, with no
+    dispatch launch; the same call with gradients on dispatches.  Both forms give the same
+    bits -- output, counts and expert ids -- at the edges of a 32-row tile and of the pairs
+    the scan takes (341 tokens x 6 = 2046; 342 dispatch), with every token on the same
+    experts (zero tokens) and spread out, with and without biases, shared experts and the
+    norm, and for more experts per token than the combine holds in registers."""
+    from nanospeaker_amd import _native as nat
+    from nanospeaker_amd.decoder import RMSNorm
+
+    for cfg in (dict(), dict(dtype=torch.float16, bias=True), dict(S=0, d=128, E=12, d_ff=96, k=4),
+                dict(S=1, d=64, E=16, d_ff=96, k=10)):
+        m, _, x, _ = build(T, **cfg)
+        m, x = m.to(DEV).eval(), x.to(DEV)
+        if collapsed:
+            x = torch.zeros_like(x)
+        norm = RMSNorm(x.shape[1]).to(DEV, x.dtype)
+        for call in (m, lambda t: m.forward_residual(t, norm)):
+            ref = call(x).detach()
+            want = (ref, m.expert_counts.clone(), m._routing.clone(), m.aux_loss.clone())
+            with torch.no_grad():
+                m.aux_loss = None
+                n0 = nat.launch_count()
+                out = call(x)
+                n1 = nat.launch_count()
+            got = (out, m.expert_counts, m._routing, m.aux_loss)
+            for name, u, v in zip(("out", "counts", "ids", "aux"), got, want):
+                assert torch.equal(u, v), f"{name} cfg={cfg}"
+            if not cfg:  # router, experts, combine; past the scan a dispatch launch too
+                assert n1 - n0 == (3 if 6 * T <= 2048 else 4), (T, n1 - n0)
+
+
 @pytest.mark.parametrize("T", [1, 15, 17, 31, 33, 49])
 def test_fp32_tile_edges(T):
     """fp32's 32-row tiles: groups of every remainder of a tile (the shared groups hold all T
