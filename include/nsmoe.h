@@ -419,6 +419,15 @@ typedef struct nsmoe_attn_args {
 
 int nsmoe_attn_prefill(const nsmoe_attn_args* args, void* stream);
 
+/* out [n_rows, n] = x [n_rows, k] W (+ resid [n_rows, n], may be out itself): the dense
+ * projections on either side of the prefill attention (the fused Q/K/V projection and W_O with
+ * the residual, mha.py:245-287), 16-bit types, fp32 accumulation, one rounding.  w_packed is W
+ * [k, n] in MFMA fragment order, [n / 16][k / 32][lane][8] with lane = (row % 32) / 8 * 16 +
+ * column % 16 and element row % 8.  k % 32 == 0, k <= 576, n % 16 == 0; contiguous rows,
+ * 16-byte aligned pointers. */
+int nsmoe_linear(int32_t dtype, const void* x, int64_t n_rows, int32_t k, int32_t n,
+                 const void* w_packed, const void* resid, void* out, void* stream);
+
 /* ---- cross-entropy over the tied head's logits ----------------------------------------
  * The loss part of NanoSpeaker.forward with targets (src/model/nanospeaker.py:236-250:
  * F.cross_entropy((h @ embed.weight.T).float(), y), mean over the targets that are not

@@ -105,6 +105,7 @@ SIGNATURES = {
     "nsmoe_rms_norm": (ctypes.c_int, [_i32, _vp, _vp, ctypes.c_float, _i64, _i32, _vp, _vp,
                                       _vp]),
     "nsmoe_attn_prefill": (ctypes.c_int, [ctypes.POINTER(AttnArgs), _vp]),
+    "nsmoe_linear": (ctypes.c_int, [_i32, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp]),
     "nsmoe_cross_entropy_rows": (ctypes.c_int, [_i32, _vp, _i64, _i64, _i32, _vp, _i64, _vp,
                                                 _vp, _vp, _vp]),
 }

@@ -21,16 +21,9 @@
 
 namespace nsmoe {
 
-// One 16-row block of a wave's 48-column slice of a 192-column pass, from the packed MFMA
-// accumulators: lo[j] / hi[j] hold columns cw + 16 j + 4 lg .. + 1 / + 2 .. + 3 of row
-// row0 + lc (lane 16 lg + lc).  Blocks 0 and 1 are regrouped across lanes (two permlane
-// swaps per dword) so that lane (lc, lg) holds columns cw + 8 lg .. + 7 of its row;
-// permlane32_swap(b0, b1) gives rows (b0.r0, b0.r1, b1.r0, b1.r1) and (b0.r2, b0.r3, b1.r2,
-// b1.r3), permlane16_swap of those (b0.r0, b0.r2, b1.r0, b1.r2) and (b0.r1, b0.r3, b1.r1,
-// b1.r3).  That 64-byte row segment and block 2's 32 bytes (columns cw + 32 + 4 lg ..) are
-// then moved to the quad-major lane order (bperm_to_quads), so each quad of lanes writes
-// one row's contiguous bytes: a 16-byte store and an 8-byte store per lane.  cw is
-// wave-uniform; rows at or past `rows` and columns at or past d are not written.
+// One 16-row block of a wave's 48-column slice of a 192-column pass (columns cw .. + 47,
+// gemm_core.h's quad order); cw is wave-uniform; rows at or past `rows` and columns at or past
+// d are not written.  slot: the rows' places in Y (row m itself without).
 template <int DT>
 __device__ __forceinline__ void store_block48(const uint32_t (&lo)[3], const uint32_t (&hi)[3],
                                               typename Elem<DT>::T* Y, int d, int row0,
@@ -38,19 +31,9 @@ __device__ __forceinline__ void store_block48(const uint32_t (&lo)[3], const uin
                                               const int* slot = nullptr) {
   using T = typename Elem<DT>::T;
   if (cw + 32 <= d) {
-    const auto l32 = __builtin_amdgcn_permlane32_swap(lo[0], lo[1], false, false);
-    const auto h32 = __builtin_amdgcn_permlane32_swap(hi[0], hi[1], false, false);
-    const auto l16 = __builtin_amdgcn_permlane16_swap(l32[0], l32[1], false, false);
-    const auto h16 = __builtin_amdgcn_permlane16_swap(h32[0], h32[1], false, false);
-    const int qa = bperm_to_quads(lane);
-    const u32x4 v = bperm4(qa, u32x4{l16[0], h16[0], l16[1], h16[1]});
-    const uint32_t b2lo = bperm(qa, lo[2]), b2hi = bperm(qa, hi[2]);
-    const int m = row0 + (lane >> 2), c = lane & 3;
-    if (m < rows) {
-      T* yrow = Y + (int64_t)(slot ? slot[m] : m) * d;
-      *(u32x4*)(yrow + cw + c * 8) = v;
-      if (cw + 32 < d) *(uint2*)(yrow + cw + 32 + c * 4) = make_uint2(b2lo, b2hi);
-    }
+    const int m = row0 + (lane >> 2);
+    T* yrow = m < rows ? Y + (int64_t)(slot ? slot[m] : m) * d + cw : nullptr;
+    store_quads48(lo, hi, (char*)yrow, lane, cw + 32 < d);
   } else if (cw < d) {
     const int m = row0 + (lane & 15);
     if (m < rows)

@@ -298,6 +298,53 @@ __device__ __forceinline__ u32x4 bperm4(int addr, const u32x4& v) {
   return u32x4{bperm(addr, v[0]), bperm(addr, v[1]), bperm(addr, v[2]), bperm(addr, v[3])};
 }
 
+// One 16-row x 48-column block of a row-major 16-bit matrix, from the packed MFMA
+// accumulators: lo[j] / hi[j] of lane 16 q + r hold columns 16 j + 4 q, + 1 / + 2, + 3 of row
+// r.  Blocks 0 and 1 are regrouped across lanes (two permlane swaps per dword) so that lane
+// (r, q) holds columns 8 q .. + 7 of its row; permlane32_swap(b0, b1) gives rows (b0.r0,
+// b0.r1, b1.r0, b1.r1) and (b0.r2, b0.r3, b1.r2, b1.r3), permlane16_swap of those (b0.r0,
+// b0.r2, b1.r0, b1.r2) and (b0.r1, b0.r3, b1.r1, b1.r3).  That 64-byte row segment and block
+// 2's 32 bytes are then moved to the quad-major order, so each quad of lanes writes one
+// row's contiguous bytes: a 16-byte store and (with `third`) an 8-byte store per lane.
+// yrow: column 0 of the block in row lane / 4, NULL for a row that is not written.
+__device__ __forceinline__ void store_quads48(const uint32_t (&lo)[3], const uint32_t (&hi)[3],
+                                              char* yrow, int lane, bool third) {
+  const auto l32 = __builtin_amdgcn_permlane32_swap(lo[0], lo[1], false, false);
+  const auto h32 = __builtin_amdgcn_permlane32_swap(hi[0], hi[1], false, false);
+  const auto l16 = __builtin_amdgcn_permlane16_swap(l32[0], l32[1], false, false);
+  const auto h16 = __builtin_amdgcn_permlane16_swap(h32[0], h32[1], false, false);
+  const int qa = bperm_to_quads(lane);
+  const u32x4 v = bperm4(qa, u32x4{l16[0], h16[0], l16[1], h16[1]});
+  const uint32_t b2lo = bperm(qa, lo[2]), b2hi = bperm(qa, hi[2]);
+  if (yrow) {
+    *(u32x4*)(yrow + (lane & 3) * 16) = v;
+    if (third) *(uint2*)(yrow + 64 + (lane & 3) * 8) = make_uint2(b2lo, b2hi);
+  }
+}
+
+// Its inverse: the same block read quad-major into the accumulators' lane order.
+__device__ __forceinline__ void load_quads48(uint32_t (&lo)[3], uint32_t (&hi)[3],
+                                             const char* yrow, int lane, bool third) {
+  u32x4 v = {0u, 0u, 0u, 0u};
+  uint2 b2 = make_uint2(0u, 0u);
+  if (yrow) {
+    v = *(const u32x4*)(yrow + (lane & 3) * 16);
+    if (third) b2 = *(const uint2*)(yrow + 64 + (lane & 3) * 8);
+  }
+  const int fa = bperm_from_quads(lane);
+  const u32x4 u = bperm4(fa, v);
+  lo[2] = bperm(fa, b2.x);
+  hi[2] = bperm(fa, b2.y);
+  const auto l16 = __builtin_amdgcn_permlane16_swap(u[0], u[2], false, false);
+  const auto h16 = __builtin_amdgcn_permlane16_swap(u[1], u[3], false, false);
+  const auto l32 = __builtin_amdgcn_permlane32_swap(l16[0], l16[1], false, false);
+  const auto h32 = __builtin_amdgcn_permlane32_swap(h16[0], h16[1], false, false);
+  lo[0] = l32[0];
+  lo[1] = l32[1];
+  hi[0] = h32[0];
+  hi[1] = h32[1];
+}
+
 // ---- fp32 row operands in the quad order ----
 //
 // A row-major fp32 operand (column n0 + r of the fragment is row(n0 + r), k contiguous, 32 of

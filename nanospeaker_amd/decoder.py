@@ -8,8 +8,8 @@ The FFN half of each block, x + moe(norm_ffn(x)), runs through MoEBlock.forward_
 which takes the RMSNorm and the residual add into the block's HIP kernels.  The attention
 of a gradient-free 16-bit forward on the GPU (the prefill) runs through `attn_prefill`,
 the library's HIP kernels (nsmoe_attn_prefill: QK-norm, RoPE, windowed or full causal
-grouped-query flash attention) between two torch GEMMs, the fused Q/K/V projection and
-W_O.  Everywhere else (CPU, fp32 / fp64, a forward that autograd differentiates, or
+grouped-query flash attention) between the fused Q/K/V projection and W_O with the residual,
+which run on nsmoe_linear for the shapes it takes and in torch otherwise.  Everywhere else (CPU, fp32 / fp64, a forward that autograd differentiates, or
 `kernel=False`) the attention is plain PyTorch: `F.rms_norm`, the rotation in the dtype
 and `scaled_dot_product_attention` (the reference's SDPA path, `flex=False`); that path is
 also the GPU kernel's reference in the tests.  The stack runs the prefill of the
@@ -133,6 +133,12 @@ def _as(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     return t.detach().to(dtype).contiguous()
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """t contiguous at a 16-byte aligned address (itself, or a copy)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """F.rms_norm(x, (d,), w, eps) of a contiguous 16-bit GPU tensor on the library's kernel
     (nsmoe_rms_norm).  Forward only."""
@@ -143,6 +149,32 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
                                        float(eps), x.numel() // d, d, y.data_ptr(), None,
                                        _stream()), "nsmoe_rms_norm")
     return y
+
+
+def pack_linear(w: torch.Tensor) -> torch.Tensor:
+    """A weight [k, n] (k % 32 == 0, n % 16 == 0) in the fragment order nsmoe_linear reads:
+    [n / 16][k / 32][(row % 32) / 8][column % 16][row % 8]."""
+    k, n = w.shape
+    return w.detach().reshape(k // 32, 4, 8, n // 16, 16).permute(3, 0, 1, 4, 2).contiguous()
+
+
+def linear_supported(k: int, n: int) -> bool:
+    """The shapes nsmoe_linear takes."""
+    return k % 32 == 0 and 32 <= k <= 576 and n % 16 == 0 and n <= 65536
+
+
+def linear(x: torch.Tensor, w_packed: torch.Tensor, n: int,
+           resid: "torch.Tensor | None" = None, out: "torch.Tensor | None" = None) -> torch.Tensor:
+    """x [rows, k] W (+ resid [rows, n]) on the library's kernel (nsmoe_linear), W packed by
+    pack_linear; `out` may be resid itself.  Contiguous 16-bit GPU tensors; forward only."""
+    rows, k = x.shape
+    if out is None:
+        out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
+    nat.check(nat.lib().nsmoe_linear(_ATTN_DT[x.dtype], x.data_ptr(), rows, k, n,
+                                     w_packed.data_ptr(),
+                                     None if resid is None else resid.data_ptr(),
+                                     out.data_ptr(), _stream()), "nsmoe_linear")
+    return out
 
 
 def attn_prefill(qkv: torch.Tensor, B: int, T: int, n_heads: int, n_kv_heads: int,
@@ -236,6 +268,7 @@ class Attention(nn.Module):
         self.W_O = nn.Parameter(torch.randn(h * dh, d) * cfg.std / math.sqrt(2 * cfg.n_layers))
         self.q_norm = RMSNorm(dh, cfg.norm_eps)
         self.k_norm = RMSNorm(dh, cfg.norm_eps)
+        self._packs: dict = {}  # _packed
 
     def use_kernel(self, z: torch.Tensor) -> bool:
         """The HIP prefill kernels take a gradient-free 16-bit forward on the GPU with
@@ -245,59 +278,61 @@ class Attention(nn.Module):
                 and not (torch.is_grad_enabled() and any(
                     t.requires_grad for t in (z, self.W_q, self.W_k, self.W_v, self.W_O))))
 
-    def _w_qkv(self, dtype) -> torch.Tensor:
-        """[W_q | W_k | W_v] in `dtype`, kept while the three weights are unchanged (their
-        identity, storage and autograd versions)."""
-        key = tuple((t.data_ptr(), t._version) for t in (self.W_q, self.W_k, self.W_v))
-        key += (dtype,)
-        hit = getattr(self, "_qkv_cache", None)
+    def _packed(self, name: str, dtype, *weights) -> torch.Tensor:
+        """The weights side by side, packed for nsmoe_linear in `dtype`, kept while they are
+        unchanged (their storage, shape and autograd versions).  A shape the kernel does not
+        take is kept as the plain matrix."""
+        key = tuple((t.data_ptr(), t._version, t.shape, t.stride()) for t in weights) + (dtype,)
+        hit = self._packs.get(name)
         if hit is None or hit[0] != key:
-            w = torch.cat((self.W_q, self.W_k, self.W_v), dim=1).to(dtype).detach()
-            hit = self._qkv_cache = (key, w)
+            w = torch.cat(weights, dim=1) if len(weights) > 1 else weights[0]
+            w = w.detach().to(dtype)
+            hit = self._packs[name] = (key, pack_linear(w) if linear_supported(*w.shape) else w)
         return hit[1]
 
-    def _w_o_t(self, dtype) -> torch.Tensor:
-        """W_O in `dtype` as the transpose of a contiguous [d, h dh] copy, kept while W_O is
-        unchanged: the library's GEMM of the residual update, x + o W_O, runs faster with
-        that operand layout (47 against 53 us at the prefill's 32,768 x 576 x 576)."""
-        key = (self.W_O.data_ptr(), self.W_O._version, dtype)
-        hit = getattr(self, "_wo_cache", None)
-        if hit is None or hit[0] != key:
-            w = self.W_O.detach().to(dtype).t().contiguous()
-            hit = self._wo_cache = (key, w)
-        return hit[1].t()
+    def _project(self, x: torch.Tensor, name: str, n: int, *weights, resid=None, out=None):
+        """x [rows, k] @ [weights] (+ resid) on nsmoe_linear, or torch for other shapes."""
+        w = self._packed(name, x.dtype, *weights)
+        if w.dim() == 5:  # packed
+            if out is not None and out.data_ptr() % 16:
+                return out.copy_(linear(_aligned(x), w, n, _aligned(resid)))
+            return linear(_aligned(x), w, n, None if resid is None else _aligned(resid), out)
+        if resid is None:
+            return x @ w
+        return torch.addmm(resid, x, w) if out is None else out.addmm_(x, w)
 
     def _kernel_attention(self, z: torch.Tensor) -> torch.Tensor:
         """[B T, h dh]: the attention output before W_O, on the HIP prefill kernels."""
         B, T, _ = z.shape
-        qkv = z.reshape(B * T, -1) @ self._w_qkv(z.dtype)
+        qkv = self._project(z.reshape(B * T, -1), "qkv", (self.h + 2 * self.hk) * self.dh,
+                            self.W_q, self.W_k, self.W_v)
         cos, sin = self.rotary.tables_f32(T, z.device)
         return attn_prefill(qkv, B, T, self.h, self.hk, self.q_norm.gamma, self.k_norm.gamma,
                             cos, sin, self.window, self.q_norm.eps)
 
     def forward_residual(self, x: torch.Tensor, z: torch.Tensor,
                          inplace: bool = False) -> torch.Tensor:
-        """x + self(z): on the kernel path the residual enters the W_O GEMM as its addend
+        """x + self(z): on the kernel path the residual enters the W_O product as its addend
         (one rounding of x + o W_O instead of two); elsewhere exactly x + self(z).  With
         `inplace` (a caller that owns x and needs it no more) the kernel path accumulates
-        into x's own memory and returns x, which saves the library GEMM's copy of the
-        addend (37.7 MB at the prefill's 32,768 x 576)."""
+        into x's own memory and returns x."""
         if self.use_kernel(z) and x.dtype == z.dtype and not (
                 torch.is_grad_enabled() and x.requires_grad):
             B, T, d = x.shape
             o = self._kernel_attention(z)
-            w = self._w_o_t(z.dtype)
             if inplace and x.is_contiguous():
-                x.view(B * T, d).addmm_(o, w)
+                xr = x.view(B * T, d)
+                self._project(o, "o", d, self.W_O, resid=xr, out=xr)
                 return x
-            return torch.addmm(x.reshape(B * T, d), o, w).view(B, T, d)
+            return self._project(o, "o", d, self.W_O,
+                                 resid=_as(x.reshape(B * T, d), x.dtype)).view(B, T, d)
         return x + self(z)
 
     def forward(self, z: torch.Tensor) -> torch.Tensor:
         B, T, _ = z.shape
         if self.use_kernel(z):
             o = self._kernel_attention(z)
-            return o.view(B, T, self.h * self.dh) @ self.W_O
+            return self._project(o, "o", self.W_O.shape[1], self.W_O).view(B, T, -1)
         q = (z @ self.W_q).view(B, T, self.h, self.dh).transpose(1, 2)
         k = (z @ self.W_k).view(B, T, self.hk, self.dh).transpose(1, 2)
         v = (z @ self.W_v).view(B, T, self.hk, self.dh).transpose(1, 2)

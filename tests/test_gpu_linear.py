@@ -1,0 +1,86 @@
+"""
+nsmoe_linear (nanospeaker_amd/csrc/linear.hip) against the same product in 64 bits: x W and
+x W + resid with one rounding of the fp32 sum, at the edges of its row tiles (32, 64 and 128 rows) and of the row counts that choose them,
+of a wave's 48, 32 and 16 columns and of a pass of 576, and through the attention sublayer
+with operands the kernel cannot read in place.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+pytest.importorskip("nanospeaker_amd.moe_kernel")
+from nanospeaker_amd import _native as nat  # noqa: E402
+from nanospeaker_amd.decoder import (Attention, DecoderConfig, Rotary, linear,  # noqa: E402
+                                     pack_linear)
+
+DEV = "cuda"
+
+
+def _operands(M, K, N, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(M, K, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(K, N, generator=g) * 0.05).to(dtype).to(DEV)
+    r = torch.randn(M, N, generator=g).to(dtype).to(DEV)
+    return x, w, r
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [
+    (1, 576, 960), (31, 576, 960), (33, 576, 576), (127, 64, 16), (129, 32, 48), (300, 544, 592),
+    (4097, 576, 960), (8193, 576, 576), (12289, 576, 960), (16385, 576, 576), (28800, 576, 576), (28673, 96, 976), (500, 576, 1152),
+    (77, 320, 1328)])
+def test_linear_against_64_bits(M, K, N, dtype):
+    """A result is one rounding of an fp32 sum: within the dtype's unit roundoff (2^-8 for
+    bf16's 8 significant bits, 2^-11 for fp16's 11) of the exact one plus the sum's own error, K
+    terms of 2^-24 of their magnitude sum.  In place (out = resid) and without a residual."""
+    x, w, r = _operands(M, K, N, dtype, M + N)
+    print(f"[linear] {M} x {K} x {N} {dtype}", flush=True)
+    wp = pack_linear(w)
+    step = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
+    xd, wd = x.double(), w.double()
+    mags = xd.abs() @ wd.abs()
+    for resid in (None, r):
+        ref = xd @ wd + (0 if resid is None else r.double())
+        bound = ref.abs() * step * 1.01 + (mags + (0 if resid is None else r.double().abs())) * (
+            K * 2.0 ** -24) + 1e-7
+        got = linear(x, wp, N, resid)
+        assert ((got.double() - ref).abs() <= bound).all()
+    acc = r.clone()
+    out = linear(x, wp, N, acc, acc)
+    assert out.data_ptr() == acc.data_ptr() and torch.equal(out, got)
+
+
+def test_linear_rejects_what_it_does_not_take():
+    x, w, r = _operands(8, 64, 32, torch.bfloat16, 0)
+    wp = pack_linear(w)
+    args = lambda k=64, n=32, out=r: (nat.BF16, x.data_ptr(), 8, k, n, wp.data_ptr(), None,
+                                      out.data_ptr(), None)
+    for bad in (args(k=48), args(k=608), args(n=24), args(out=r.view(-1)[1:])):
+        assert nat.lib().nsmoe_linear(*bad) == 1
+    assert nat.lib().nsmoe_linear(nat.F32, *args()[1:]) == 1
+    assert nat.lib().nsmoe_linear(nat.BF16, None, 0, 64, 32, None, None, None, None) == 0
+
+
+@pytest.mark.parametrize("d_model", [576, 584])
+def test_attention_sublayer_operands(d_model):
+    """forward_residual with strided, misaligned and in-place operands, and with a d_model the
+    kernel does not take (584: torch products), all equal to the plain call; an in-place
+    weight update is seen."""
+    torch.manual_seed(0)
+    cfg = DecoderConfig(d_model=d_model)
+    att = Attention(cfg, Rotary(64, cfg.rope_base), None).to(DEV, torch.bfloat16).eval()
+    x = torch.randn(2, 70, d_model, device=DEV, dtype=torch.bfloat16)
+    z = torch.randn_like(x)
+    odd = lambda t: torch.cat((t.new_zeros(1), t.reshape(-1)))[1:].view(t.shape)
+    with torch.no_grad():
+        ref = att.forward_residual(x, z)
+        assert torch.equal(att.forward_residual(x, z.transpose(0, 1).contiguous().transpose(0, 1)),
+                           ref)
+        assert torch.equal(att.forward_residual(odd(x), odd(z)), ref)
+        for own in (x.clone(), odd(x)):
+            got = att.forward_residual(own, z, inplace=True)
+            assert got.data_ptr() == own.data_ptr() and torch.equal(got, ref)
+        att.W_O.mul_(2.0)
+        assert not torch.equal(att.forward_residual(x, z), ref)
