@@ -227,6 +227,20 @@ extern "C" uint64_t nsmoe_launch_count(void) {
   return nsmoe::g_launches.load(std::memory_order_relaxed);
 }
 
+int nsmoe::device_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        n <= 0)
+      n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 extern "C" int32_t nsmoe_abi_version(void) { return 8; }
 
 extern "C" int nsmoe_set_option(const char* name, int64_t value) {

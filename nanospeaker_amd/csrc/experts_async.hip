@@ -1644,7 +1644,6 @@ __global__ void __launch_bounds__(NT, 3) expert_dx_res_kernel(ExpParams p) {
   wait_vmcnt<0>();
 }
 
-static int device_cus();
 static int64_t tile_grid(const ExpParams& p, int bm);
 
 template <int DT, int MB, bool SA>
@@ -2111,21 +2110,6 @@ int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_ou
   else go(std::integral_constant<int, DT_F32>{});
   timer.stop();
   return check_launch("dw_pair_kernel");
-}
-
-// Compute units of the current device (cached per device).
-static int device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-      n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
 }
 
 // Upper bound on the token tiles of `bm` rows over all groups (routed, then shared).

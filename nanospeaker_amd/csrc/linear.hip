@@ -161,21 +161,6 @@ __global__ void __launch_bounds__(LN_THREADS, 3) linear_kernel(LinearArgs a) {
   }
 }
 
-// Compute units of the current device (cached per device).
-static int device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-      n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 template <int DT>
 static int linear_launch(const LinearArgs& a, hipStream_t s) {
   // The smallest row tile whose workgroups (one per CU) still fit one round of the chip, so

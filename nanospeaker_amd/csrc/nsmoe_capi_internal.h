@@ -16,6 +16,8 @@ enum Status : int { NSMOE_OK = 0, NSMOE_EINVAL = 1, NSMOE_EHIP = 2, NSMOE_EWORKS
 
 void set_error(const char* fmt, ...);
 void note_launch();
+// Compute units of the current device (cached per device).
+int device_cus();
 
 // Checks the launch that was just enqueued; records an error string on failure.
 inline int check_launch(const char* what) {

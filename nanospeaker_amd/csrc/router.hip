@@ -537,13 +537,11 @@ static void launch_fwd(const RouterArgs& a, unsigned grid, int waves, hipStream_
   }
 }
 
-static int router_device_cus();
-
 // 8-wave workgroups (two per CU) once the grid has more workgroups than CUs, else 16
 // (one per CU, W_r copied whole); the "router_waves" option forces either.
 static int router_waves_for(int64_t grid) {
   if (const int64_t v = option(OPT_ROUTER_WAVES)) return (int)v;
-  return grid > router_device_cus() ? 8 : 16;
+  return grid > device_cus() ? 8 : 16;
 }
 
 // At most 8 pack items per packing wave: about the length of the selection and the exact
@@ -552,21 +550,6 @@ bool router_fused_can_pack(int64_t T, int64_t items) {
   const int64_t grid = router_fused_chunks(T);
   return T > 0 && router_waves_for(grid) == 16 && items <= grid * RT_PACK_WAVES * 8 &&
          !option(OPT_PACK_IN_PLACE);
-}
-
-// Compute units of the current device (cached per device).
-static int router_device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-      n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
 }
 
 int router_fused_launch(const RouterArgs& a, int dtype, hipStream_t s) {
