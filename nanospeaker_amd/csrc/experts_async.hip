@@ -1387,7 +1387,10 @@ __global__ void __launch_bounds__(NT, D > 2 || MB == 6 ? 3 : 2) expert_dx_reg_ke
   __shared__ __attribute__((aligned(16))) char s_y[STAGE_Y ? TM * Y_PITCH : 16];
   __shared__ int s_loc[3];
 
-  const int tile = tile_of_block(p);
+  // p.dx_split > 1: a workgroup takes one of the tile's passes over the output columns.
+  const int item = p.xcd_run > 0 ? xcd_deal(blockIdx.x, gridDim.x, p.xcd_run * p.dx_split)
+                                 : xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = item / p.dx_split, pass0 = item - tile * p.dx_split;
   Located loc;
   if (!locate(tile, p.E + p.S, [&](int g) { return (rows_of(p, g) + TM - 1) / TM; },
               [](int) { return 0; }, s_loc, loc))
@@ -1404,7 +1407,7 @@ __global__ void __launch_bounds__(NT, D > 2 || MB == 6 ? 3 : 2) expert_dx_reg_ke
   const int fq = bperm_from_quads(lane);
   const int nkk = twoH / G::KC;  // <= KMAX in the resident-tile kernel (the launcher checks)
   const int npass = (d + NP2 - 1) / NP2;
-  const int nsteps = npass * nkk;
+  const int nsteps = p.dx_split > 1 ? nkk : npass * nkk;
 
   struct WSet {
     Frag f[NBF];
@@ -1412,7 +1415,7 @@ __global__ void __launch_bounds__(NT, D > 2 || MB == 6 ? 3 : 2) expert_dx_reg_ke
   // W_in fragments in the quad-major lane order (lane 4 r + q: row 16 block + r, 16-byte
   // chunk q of the k-step), moved to the MFMA order with ds_bpermute when the step runs.
   auto load_w = [&](int s) __attribute__((always_inline)) -> WSet {
-    const int pass = s / nkk, k0 = (s - pass * nkk) * G::KC;
+    const int sp = s / nkk, pass = pass0 + sp, k0 = (s - sp * nkk) * G::KC;
     WSet w;
 #pragma unroll
     for (int j = 0; j < NBF; ++j) {
@@ -1452,7 +1455,7 @@ __global__ void __launch_bounds__(NT, D > 2 || MB == 6 ? 3 : 2) expert_dx_reg_ke
   T* DX = (T*)p.dxrow + slot0 * d;
   f32x4 acc[MB][3];
   auto step = [&](int s, const WSet& w) __attribute__((always_inline)) {
-    const int pass = s / nkk, kk = s - pass * nkk;
+    const int sp = s / nkk, pass = pass0 + sp, kk = s - sp * nkk;
     if (kk == 0) {
 #pragma unroll
       for (int i = 0; i < MB; ++i)
@@ -1691,9 +1694,18 @@ static void dx_reg_launch(const ExpParams& p, int mb, int dist, hipStream_t s) {
     else if (dist == 3) expert_dx_res_kernel<DT, 3><<<g6, NT, 0, s>>>(p);
     else expert_dx_res_kernel<DT, 2><<<g6, NT, 0, s>>>(p);
   } else {
-    if (dist == 4) expert_dx_reg_kernel<DT, 4, 4><<<g4, NT, 0, s>>>(p);
-    else if (dist == 3) expert_dx_reg_kernel<DT, 3, 4><<<g4, NT, 0, s>>>(p);
-    else expert_dx_reg_kernel<DT, 2, 4><<<g4, NT, 0, s>>>(p);
+    // 64-row tiles are for calls whose tiles do not fill the chip (T below ~5000 here): a
+    // workgroup per pass instead of one for all of them divides a tile's chain of k-steps
+    // by three and copies nothing twice (this kernel copies its rows for every pass anyway).
+    // expert_dx 20.4 -> 11.4 us at T = 150, 22.3 -> 16.0 at 1024, 26.9 -> 21.7 at 2047, 33.8
+    // -> 32.0 at 4096, 42.2 -> 42.5 at 6000.  The k loop unrolls by the prefetch distance.
+    ExpParams q = p;
+    const int npass = (p.d + NP2 - 1) / NP2, nkk = 2 * p.H / 32;
+    q.dx_split = nkk % dist == 0 ? npass : 1;
+    const unsigned g = g4 * (unsigned)q.dx_split;
+    if (dist == 4) expert_dx_reg_kernel<DT, 4, 4><<<g, NT, 0, s>>>(q);
+    else if (dist == 3) expert_dx_reg_kernel<DT, 3, 4><<<g, NT, 0, s>>>(q);
+    else expert_dx_reg_kernel<DT, 2, 4><<<g, NT, 0, s>>>(q);
   }
 }
 
@@ -2143,14 +2155,15 @@ static void fwd_reg_launch(const ExpParams& p, int mb, int dist, hipStream_t s) 
   }
 }
 
-// Row blocks of the register-tiled forward's tiles: 96 rows once 64-row tiles overflow the
-// resident workgroup slots (3 per CU); 32 rows (at prefetch distance 6) while 64-row tiles
-// would fill under half the CUs (decode-sized calls: a tile's time is its weight stream's
-// latency, not its rows).  The "fwd_rows" option forces a tile height.
+// Row blocks of the register-tiled forward's tiles.  32 rows (at prefetch distance 6) while
+// such tiles fit one round of their two workgroups per CU: a tile's time is then its weight
+// stream's latency, not its rows (T = 512: 19.1 us against 24.1 with 64 rows, 1531: 22.5 / 24.3;
+// 2047, past one round: 32.5 / 26.6).  96 rows once 64-row tiles overflow three per CU (6000:
+// 42.5 / 48.3; 4096, before: 35.2 / 33.7).  The "fwd_rows" option forces a tile height.
 static int fwd_row_blocks(const ExpParams& p) {
   if (const int64_t v = option(OPT_FWD_ROWS)) return (int)(v / 16);
-  const int64_t g64 = tile_grid(p, 64);
-  return g64 > 3 * (int64_t)device_cus() ? 6 : 2 * g64 <= device_cus() ? 2 : 4;
+  const int64_t cus = device_cus();
+  return tile_grid(p, 64) > 3 * cus ? 6 : tile_grid(p, 32) <= 2 * cus ? 2 : 4;
 }
 
 // d and the step counts the register-tiled forward unrolls by.

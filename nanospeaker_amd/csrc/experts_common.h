@@ -33,6 +33,7 @@ struct ExpParams {
   // Token-tile kernels: runs of xcd_run consecutive tiles are dealt round-robin over the
   // XCDs (0: each XCD takes one contiguous eighth of the grid).
   int xcd_run;
+  int dx_split;  // workgroups a dX tile's passes are split over (1 or the number of passes)
   // fragment-order weight packs (pack.hip): W_in for GEMM1, W_out for GEMM2
   const char* p_in;
   const char* p_out;

@@ -264,6 +264,19 @@ def test_dw_chunk_edges(T, dtype):
     run_case(T, train=True, backward=True, d=128, E=8, d_ff=96, k=4, S=1, dtype=dtype)
 
 
+@pytest.mark.parametrize("T", [15, 63, 65, 400])
+@pytest.mark.parametrize("cfg", [dict(), dict(d=320, E=12, k=3, S=1, d_ff=192),
+                                 dict(d=384, E=10, k=2, S=0, d_ff=144), dict(d=128, E=6, k=2, S=2,
+                                                                             d_ff=96)])
+def test_dx_passes_split_over_workgroups(T, cfg):
+    """Small calls give every pass of 192 dX columns a workgroup of its own: three passes, two
+    with a ragged second one (d 320), an odd number of k-steps (H 96, two of three 64-row
+    steps: not split) and a single pass, at the edges of a 64-row tile.  (Not at T = 1: with
+    two experts a token the router's gradient there is one difference of two gate gradients
+    rounded to bf16, 2^-9 of each, whose relative error has no bound of 5e-3.)"""
+    run_case(T, train=True, backward=True, **cfg)
+
+
 @pytest.mark.parametrize("collapsed", [False, True])
 @pytest.mark.parametrize("T", [1, 2, 31, 32, 33, 64, 65, 170, 341, 342])
 def test_decode_without_dispatch_matches_the_dispatched_forward(T, collapsed):
