@@ -9,8 +9,8 @@ which takes the RMSNorm and the residual add into the block's HIP kernels.  The 
 of a gradient-free 16-bit forward on the GPU (the prefill) runs through `attn_prefill`,
 the library's HIP kernels (nsmoe_attn_prefill: QK-norm, RoPE, windowed or full causal
 grouped-query flash attention) between the fused Q/K/V projection and W_O with the residual,
-which run on nsmoe_linear for the shapes it takes and in torch otherwise.  Everywhere else (CPU, fp32 / fp64, a forward that autograd differentiates, or
-`kernel=False`) the attention is plain PyTorch: `F.rms_norm`, the rotation in the dtype
+which run on nsmoe_linear for the shapes it takes and in torch otherwise.  Everywhere else
+(CPU, fp32 / fp64, a forward that autograd differentiates, or `kernel=False`) the attention is plain PyTorch: `F.rms_norm`, the rotation in the dtype
 and `scaled_dot_product_attention` (the reference's SDPA path, `flex=False`); that path is
 also the GPU kernel's reference in the tests.  The stack runs the prefill of the
 benchmark's fifth workload (batch 4 x 8192 tokens, eval, bf16) with the MoE kernels in
@@ -168,6 +168,19 @@ def linear(x: torch.Tensor, w_packed: torch.Tensor, n: int,
     """x [rows, k] W (+ resid [rows, n]) on the library's kernel (nsmoe_linear), W packed by
     pack_linear; `out` may be resid itself.  Contiguous 16-bit GPU tensors; forward only."""
     rows, k = x.shape
+    # The kernel reads and writes through these sizes alone, so every operand has to have them.
+    if w_packed.shape != (n // 16, k // 32, 4, 16, 8) or k % 32 or n % 16:
+        raise RuntimeError(f"linear: x {tuple(x.shape)} and n {n} do not fit packed weights "
+                           f"{tuple(w_packed.shape)}")
+    for t in (w_packed, resid, out):
+        if t is None:
+            continue
+        if t is not w_packed and t.shape != (rows, n):
+            raise RuntimeError(f"linear: addend or output {tuple(t.shape)}, expected {(rows, n)}")
+        if t.device != x.device or t.dtype != x.dtype or not t.is_contiguous():
+            raise RuntimeError("linear: operands must be contiguous, of one dtype and device")
+    if not (x.is_cuda and x.is_contiguous()):
+        raise RuntimeError("linear: x must be a contiguous GPU tensor")
     if out is None:
         out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
     nat.check(nat.lib().nsmoe_linear(_ATTN_DT[x.dtype], x.data_ptr(), rows, k, n,
@@ -279,15 +292,20 @@ class Attention(nn.Module):
                     t.requires_grad for t in (z, self.W_q, self.W_k, self.W_v, self.W_O))))
 
     def _packed(self, name: str, dtype, *weights) -> torch.Tensor:
-        """The weights side by side, packed for nsmoe_linear in `dtype`, kept while they are
+        """The weights side by side in `dtype`, packed for nsmoe_linear, kept while they are
         unchanged (their storage, shape and autograd versions).  A shape the kernel does not
-        take is kept as the plain matrix."""
-        key = tuple((t.data_ptr(), t._version, t.shape, t.stride()) for t in weights) + (dtype,)
-        hit = self._packs.get(name)
+        take, or a call under autocast (whose products choose their own dtype), is kept as the
+        plain matrix."""
+        auto = torch.is_autocast_enabled()
+        key = tuple((t.data_ptr(), t._version, t.shape, t.stride()) for t in weights)
+        key += (dtype, auto)
+        packs = self.__dict__.setdefault("_packs", {})  # absent in a module pickled without it
+        hit = packs.get(name)
         if hit is None or hit[0] != key:
             w = torch.cat(weights, dim=1) if len(weights) > 1 else weights[0]
             w = w.detach().to(dtype)
-            hit = self._packs[name] = (key, pack_linear(w) if linear_supported(*w.shape) else w)
+            plain = auto or not linear_supported(*w.shape)
+            hit = packs[name] = (key, w if plain else pack_linear(w))
         return hit[1]
 
     def _project(self, x: torch.Tensor, name: str, n: int, *weights, resid=None, out=None):
@@ -332,6 +350,8 @@ class Attention(nn.Module):
         B, T, _ = z.shape
         if self.use_kernel(z):
             o = self._kernel_attention(z)
+            if self.W_O.dtype != o.dtype:  # torch's rules for mixed operands
+                return o.view(B, T, self.h * self.dh) @ self.W_O
             return self._project(o, "o", self.W_O.shape[1], self.W_O).view(B, T, -1)
         q = (z @ self.W_q).view(B, T, self.h, self.dh).transpose(1, 2)
         k = (z @ self.W_k).view(B, T, self.hk, self.dh).transpose(1, 2)

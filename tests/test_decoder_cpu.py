@@ -113,3 +113,30 @@ def test_trunk_balance_loss_is_the_promoted_sum_of_the_blocks():
         assert aux.dtype == torch.float32
         assert torch.equal(aux, ref), (train, aux, ref)
         assert (float(aux) != 0.0) == train
+
+
+def test_linear_refuses_operands_that_do_not_fit():
+    """The projection kernel reads and writes through the sizes it is given, so the wrapper
+    refuses, before any launch, an addend or output of other rows, columns, dtype or layout,
+    a width the packed weights do not have, and host tensors."""
+    from nanospeaker_amd.decoder import linear, pack_linear
+
+    x, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(64, 32, dtype=torch.bfloat16)
+    wp, ok = pack_linear(w), torch.zeros(4, 32, dtype=torch.bfloat16)
+    for args in ((x, wp, 48), (x, wp, 33), (x[:, :32], wp, 32), (x, wp, 32, ok[:3]),
+                 (x, wp, 32, ok[:, :16]), (x, wp, 32, ok.float()), (x, wp, 32, ok[:1]),
+                 (x, wp, 32, torch.zeros(32, 4, dtype=torch.bfloat16).t()),
+                 (x, wp, 32, ok, ok[:3]), (x, wp, 32)):
+        with pytest.raises(RuntimeError, match="linear"):
+            linear(*args)
+
+
+def test_attention_packs_survive_a_module_saved_without_them():
+    """A module object pickled before the weights' packed copies were kept has no `_packs`."""
+    from nanospeaker_amd.decoder import Attention
+
+    cfg = DecoderConfig(d_model=64, n_heads=1, n_kv_heads=1)
+    att = Attention(cfg, Rotary(64, cfg.rope_base), None)
+    del att._packs
+    assert att._packed("o", torch.bfloat16, att.W_O).shape == (4, 2, 4, 16, 8)
+    assert len(att._packs) == 1

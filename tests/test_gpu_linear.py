@@ -84,3 +84,21 @@ def test_attention_sublayer_operands(d_model):
             assert got.data_ptr() == own.data_ptr() and torch.equal(got, ref)
         att.W_O.mul_(2.0)
         assert not torch.equal(att.forward_residual(x, z), ref)
+
+
+def test_attention_refuses_a_residual_that_does_not_fit():
+    """A residual of other rows, another width, dtype or device than the layer's output is
+    refused on the host, in place or not; W_O in another dtype than the tokens is refused by
+    the plain forward, as a torch product of mixed operands is."""
+    cfg = DecoderConfig()
+    att = Attention(cfg, Rotary(64, cfg.rope_base), None).to(DEV, torch.bfloat16).eval()
+    z = torch.randn(2, 70, 576, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        for x in (z[:, :69].contiguous(), z[:1], torch.cat((z, z), dim=-1), z[..., :64].contiguous(),
+                  z.cpu()):
+            for inplace in (False, True):
+                with pytest.raises(RuntimeError):
+                    att.forward_residual(x, z, inplace=inplace)
+        att.W_O.data = att.W_O.data.float()
+        with pytest.raises(RuntimeError):
+            att(z)
