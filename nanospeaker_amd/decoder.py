@@ -9,10 +9,11 @@ which takes the RMSNorm and the residual add into the block's HIP kernels.  The 
 of a gradient-free 16-bit forward on the GPU (the prefill) runs through `attn_prefill`,
 the library's HIP kernels (nsmoe_attn_prefill: QK-norm, RoPE, windowed or full causal
 grouped-query flash attention) between the fused Q/K/V projection and W_O with the residual,
-which run on nsmoe_linear for the shapes it takes and in torch otherwise.  Everywhere else
-(CPU, fp32 / fp64, a forward that autograd differentiates, or `kernel=False`) the attention is plain PyTorch: `F.rms_norm`, the rotation in the dtype
-and `scaled_dot_product_attention` (the reference's SDPA path, `flex=False`); that path is
-also the GPU kernel's reference in the tests.  The stack runs the prefill of the
+which run on nsmoe_linear for the shapes it takes and in torch otherwise (`Attention.forward`,
+which adds no residual, multiplies by W_O in torch).  Everywhere else (CPU, fp32 / fp64, a
+forward that autograd differentiates, or `kernel=False`) the attention is plain PyTorch:
+`F.rms_norm`, the rotation in the dtype and `scaled_dot_product_attention` (the reference's
+SDPA path, `flex=False`); that path is also the GPU kernel's reference in the tests.  The stack runs the prefill of the
 benchmark's fifth workload (batch 4 x 8192 tokens, eval, bf16) with the MoE kernels in
 situ, so the block's share of a real forward can be measured.
 
@@ -349,10 +350,10 @@ class Attention(nn.Module):
     def forward(self, z: torch.Tensor) -> torch.Tensor:
         B, T, _ = z.shape
         if self.use_kernel(z):
+            # W_O as it is now, by torch's product: no packed copy that a write through
+            # `.data` would leave behind, and torch's rules for mixed operands.
             o = self._kernel_attention(z)
-            if self.W_O.dtype != o.dtype:  # torch's rules for mixed operands
-                return o.view(B, T, self.h * self.dh) @ self.W_O
-            return self._project(o, "o", self.W_O.shape[1], self.W_O).view(B, T, -1)
+            return o.view(B, T, self.h * self.dh) @ self.W_O
         q = (z @ self.W_q).view(B, T, self.h, self.dh).transpose(1, 2)
         k = (z @ self.W_k).view(B, T, self.hk, self.dh).transpose(1, 2)
         v = (z @ self.W_v).view(B, T, self.hk, self.dh).transpose(1, 2)

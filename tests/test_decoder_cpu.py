@@ -140,3 +140,40 @@ def test_attention_packs_survive_a_module_saved_without_them():
     del att._packs
     assert att._packed("o", torch.bfloat16, att.W_O).shape == (4, 2, 4, 16, 8)
     assert len(att._packs) == 1
+
+
+def _kernel_path_on_the_cpu(monkeypatch, att, o):
+    """The module's kernel path with its launches replaced: the attention's output is `o`,
+    and the projection kernel is a torch product by the unpacked weights."""
+    from nanospeaker_amd import decoder as D
+
+    def linear(x, w_packed, n, resid=None, out=None):
+        nb, kb = w_packed.shape[:2]
+        y = x @ w_packed.permute(1, 2, 4, 0, 3).reshape(kb * 32, nb * 16)
+        y = y if resid is None else y + resid
+        return y if out is None else out.copy_(y)
+
+    monkeypatch.setattr(D, "linear", linear)
+    monkeypatch.setattr(att, "use_kernel", lambda z: True)
+    monkeypatch.setattr(att, "_kernel_attention", lambda z: o)
+
+
+def _small_attention():
+    from nanospeaker_amd.decoder import Attention
+
+    cfg = DecoderConfig(d_model=64, n_heads=1, n_kv_heads=1)
+    return Attention(cfg, Rotary(64, cfg.rope_base), None).eval()
+
+
+def test_plain_attention_reads_the_current_output_weight(monkeypatch):
+    """Attention.forward multiplies by W_O as it is at the call, also after writes that the
+    version counter does not see and after the parameter was replaced at the same address."""
+    att, o, z = _small_attention(), torch.randn(6, 64), torch.zeros(2, 3, 64)
+    _kernel_path_on_the_cpu(monkeypatch, att, o)
+    with torch.no_grad():
+        for _ in range(2):
+            assert torch.equal(att(z), o.view(2, 3, 64) @ att.W_O)
+            att.W_O.data.mul_(2.0)
+            assert torch.equal(att(z), o.view(2, 3, 64) @ att.W_O)
+            att.W_O.data.add_(1.0)
+            att.W_O = torch.nn.Parameter(att.W_O.data)

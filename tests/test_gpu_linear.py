@@ -102,3 +102,17 @@ def test_attention_refuses_a_residual_that_does_not_fit():
         att.W_O.data = att.W_O.data.float()
         with pytest.raises(RuntimeError):
             att(z)
+
+
+def test_plain_attention_reads_the_current_output_weight():
+    """forward() on the kernel path is the attention's output times W_O by torch's product,
+    bit for bit, also after a write through `.data`."""
+    torch.manual_seed(1)
+    cfg = DecoderConfig()
+    att = Attention(cfg, Rotary(64, cfg.rope_base), None).to(DEV, torch.bfloat16).eval()
+    z = torch.randn(2, 70, 576, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        for _ in range(2):
+            o = att._kernel_attention(z).view(2, 70, -1)
+            assert torch.equal(att(z), o @ att.W_O)
+            att.W_O.data.mul_(2.0)
