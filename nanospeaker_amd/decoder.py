@@ -39,7 +39,7 @@ from torch import nn
 from . import _native as nat
 from .head import linear_cross_entropy
 from .moe import MoEBlock
-from .moe_kernel import _stream
+from .moe_kernel import PACKS, PackCache, _stream
 
 
 @dataclass
@@ -155,8 +155,20 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 def pack_linear(w: torch.Tensor) -> torch.Tensor:
     """A weight [k, n] (k % 32 == 0, n % 16 == 0) in the fragment order nsmoe_linear reads:
     [n / 16][k / 32][(row % 32) / 8][column % 16][row % 8]."""
+    return _fragments(w.detach()).contiguous()
+
+
+def _fragments(w: torch.Tensor) -> torch.Tensor:
     k, n = w.shape
-    return w.detach().reshape(k // 32, 4, 8, n // 16, 16).permute(3, 0, 1, 4, 2).contiguous()
+    return w.reshape(k // 32, 4, 8, n // 16, 16).permute(3, 0, 1, 4, 2)
+
+
+@torch.inference_mode()  # refresh() also writes buffers that were made in inference mode
+def _pack_projection(weights, into: torch.Tensor) -> None:
+    """The weights side by side, cast and written in place: in nsmoe_linear's order, or as the
+    plain matrix where `into` has its two dimensions."""
+    w = (torch.cat(tuple(weights), dim=1) if len(weights) > 1 else weights[0]).to(into.dtype)
+    into.copy_(w if into.dim() == 2 else _fragments(w))
 
 
 def linear_supported(k: int, n: int) -> bool:
@@ -269,6 +281,8 @@ class Attention(nn.Module):
     """Grouped-query self-attention with QK-norm, rotary embeddings and an optional window
     (reference: OptimizedMultiHeadAttention, mha.py:245-287, on its SDPA path)."""
 
+    _PACK_CAPACITY = 8  # two projections in up to two dtypes, packed and plain
+
     def __init__(self, cfg: DecoderConfig, rotary: Rotary, window: "int | None",
                  kernel: bool = True):
         super().__init__()
@@ -282,7 +296,7 @@ class Attention(nn.Module):
         self.W_O = nn.Parameter(torch.randn(h * dh, d) * cfg.std / math.sqrt(2 * cfg.n_layers))
         self.q_norm = RMSNorm(dh, cfg.norm_eps)
         self.k_norm = RMSNorm(dh, cfg.norm_eps)
-        self._packs: dict = {}  # _packed
+        self._packs = PACKS.child(self._PACK_CAPACITY)  # _packed
 
     def use_kernel(self, z: torch.Tensor) -> bool:
         """The HIP prefill kernels take a gradient-free 16-bit forward on the GPU with
@@ -293,21 +307,27 @@ class Attention(nn.Module):
                     t.requires_grad for t in (z, self.W_q, self.W_k, self.W_v, self.W_O))))
 
     def _packed(self, name: str, dtype, *weights) -> torch.Tensor:
-        """The weights side by side in `dtype`, packed for nsmoe_linear, kept while they are
-        unchanged (their storage, shape and autograd versions).  A shape the kernel does not
-        take, or a call under autocast (whose products choose their own dtype), is kept as the
-        plain matrix."""
-        auto = torch.is_autocast_enabled()
-        key = tuple((t.data_ptr(), t._version, t.shape, t.stride()) for t in weights)
-        key += (dtype, auto)
-        packs = self.__dict__.setdefault("_packs", {})  # absent in a module pickled without it
-        hit = packs.get(name)
-        if hit is None or hit[0] != key:
-            w = torch.cat(weights, dim=1) if len(weights) > 1 else weights[0]
-            w = w.detach().to(dtype)
-            plain = auto or not linear_supported(*w.shape)
-            hit = packs[name] = (key, w if plain else pack_linear(w))
-        return hit[1]
+        """The weights side by side in `dtype`, packed for nsmoe_linear, kept under PackCache's
+        rules (the same parameters, unchanged; the packing stream; graph capture; `.data`
+        writes need `PACKS.clear()`).  A shape the kernel does not take, or a call under
+        autocast (whose products choose their own dtype), gets the plain matrix.  A traced
+        call keeps nothing."""
+        auto, packs = torch.is_autocast_enabled(), None
+        if not torch.compiler.is_compiling():
+            packs = self.__dict__.get("_packs")
+            if not isinstance(packs, PackCache):  # a module pickled without one
+                packs = self._packs = PACKS.child(self._PACK_CAPACITY)
+            w = packs.find((name, dtype, auto), weights)
+            if w is not None:
+                return w
+        k, n = weights[0].shape[0], sum([w.shape[1] for w in weights])
+        plain = auto or not linear_supported(k, n)
+        w = torch.empty((k, n) if plain else (n // 16, k // 32, 4, 16, 8), dtype=dtype,
+                        device=weights[0].device)
+        _pack_projection(weights, w)
+        if packs is not None:
+            packs.file((name, dtype, auto), weights, w, _pack_projection)
+        return w
 
     def _project(self, x: torch.Tensor, name: str, n: int, *weights, resid=None, out=None):
         """x [rows, k] @ [weights] (+ resid) on nsmoe_linear, or torch for other shapes."""

@@ -250,8 +250,9 @@ def _c(t: Optional[Tensor]) -> Optional[Tensor]:
 
 class _PackEntry:
     """One cached pack: weak references to the key tensors and their states, the two
-    buffers, the stream they were packed on, what refresh() needs to pack them again, and
-    whether a captured graph reads them (then LRU eviction skips the entry)."""
+    buffers (p_out None in a child cache), the stream they were packed on, what refresh()
+    needs to pack them again, and whether a captured graph reads them (then LRU eviction
+    skips the entry)."""
 
     __slots__ = ("refs", "states", "p_in", "p_out", "stream", "handle", "spec", "pinned")
 
@@ -270,6 +271,16 @@ class _PackEntry:
             if ref() is not k or state != PackCache._state(k):
                 return False
         return True
+
+    def used_on(self, device_index) -> None:
+        """The current stream is about to read the buffers: if they were packed on another
+        one, it waits for that stream, and their memory is kept until it is done."""
+        if self.stream is not None and _stream(device_index) != self.handle:
+            cur = torch.cuda.current_stream(self.p_in.device)
+            cur.wait_stream(self.stream)
+            for p in (self.p_in, self.p_out):
+                if p is not None:
+                    p.record_stream(cur)
 
 
 class PackCache:
@@ -306,6 +317,11 @@ class PackCache:
       at replay: after an in-place weight update, call `refresh()` (it repacks every
       live entry into its own buffers, on the current stream) before replaying.  A
       capture that misses still packs inside the graph and files nothing.
+    * **Children.** A cache made with `child()` holds other packs under the same rules, each
+      filed under a name (`find`, `file`): an attention layer's projections, which go with
+      the layer.  The parent's `clear()`, `refresh()` and `share_with_graphs` hold for it
+      too, and a child whose entries are pinned is kept until `clear()`.  A copied or
+      pickled cache comes back empty, a child as one of PACKS.
     """
 
     def __init__(self, capacity: int = 64):
@@ -313,9 +329,26 @@ class PackCache:
         self.hits = 0
         self.misses = 0
         self.share_with_graphs = False
+        self._parent: "PackCache | None" = None
+        self._children: "weakref.WeakSet[PackCache]" = weakref.WeakSet()
+        self._held: "set[PackCache]" = set()  # children with entries that graphs read
         self._lock = threading.RLock()
         self._entries: "OrderedDict[tuple, _PackEntry]" = OrderedDict()
         self._local = threading.local()
+
+    def child(self, capacity: int) -> "PackCache":
+        """An empty cache that this one's clear(), refresh() and share_with_graphs cover."""
+        c = PackCache(capacity)
+        c._parent = self
+        # One lock for all of them: an entry's removal (_drop) can run at any allocation, so
+        # with a lock each, two threads could wait for each other's.
+        c._lock = self._lock
+        with self._lock:
+            self._children.add(c)
+        return c
+
+    def __reduce__(self):
+        return _empty_pack_cache, (self.capacity, self._parent is not None)
 
     @staticmethod
     def _state(t: Tensor) -> tuple:
@@ -327,7 +360,9 @@ class PackCache:
 
     def clear(self) -> None:
         with self._lock:
-            self._entries.clear()
+            for cache in (self, *self._children):
+                cache._entries.clear()
+            self._held.clear()
 
     def __len__(self) -> int:
         return len(self._entries)
@@ -368,12 +403,8 @@ class PackCache:
                         self.hits += 1
                         if capturing:
                             entry.pinned = True
-                        elif cuda and entry.stream is not None and (
-                                _stream(device.index) != entry.handle):
-                            cur = torch.cuda.current_stream(device)
-                            cur.wait_stream(entry.stream)
-                            entry.p_in.record_stream(cur)
-                            entry.p_out.record_stream(cur)
+                        elif cuda:
+                            entry.used_on(device.index)
                         return entry.p_in, entry.p_out, None
                     if not entry.pinned:
                         del self._entries[key]
@@ -388,7 +419,9 @@ class PackCache:
         key, keys = pending[0], pending[1]
         if not keys:
             return
-        spec = pending[2] if len(pending) > 2 else None
+        self._insert(key, keys, p_in, p_out, pending[2] if len(pending) > 2 else None)
+
+    def _insert(self, key, keys, p_in: Tensor, p_out: Optional[Tensor], spec) -> None:
         cb = lambda _ref, key=key: self._drop(key)
         stream = torch.cuda.current_stream(p_in.device) if p_in.is_cuda else None
         entry = _PackEntry(tuple(weakref.ref(k, cb) for k in keys),
@@ -403,6 +436,33 @@ class PackCache:
             for k in [k for k, e in self._entries.items() if not e.pinned][:max(over, 0)]:
                 del self._entries[k]
 
+    def find(self, name, weights) -> Optional[Tensor]:
+        """The buffer filed under `name`, if it was packed from these weights and they are
+        unchanged, ready for the current stream of their device; None if there is none, or
+        while a graph is captured that does not share packs."""
+        with self._lock:
+            entry = self._entries.get(name)
+            if entry is None or not entry.valid_for(weights):
+                self.misses += 1
+                return None
+            if entry.stream is not None:
+                if not torch.cuda.is_current_stream_capturing():
+                    entry.used_on(entry.p_in.device.index)
+                elif not self._parent.share_with_graphs:
+                    self.misses += 1
+                    return None
+                else:
+                    entry.pinned = True
+                    self._parent._held.add(self)
+            self.hits += 1
+            return entry.p_in
+
+    def file(self, name, weights, buffer: Tensor, pack) -> None:
+        """Keep `buffer`, just packed from `weights` on the current stream, under `name`,
+        unless the stream is being captured.  pack(weights, buffer) packs it again."""
+        if not (buffer.is_cuda and torch.cuda.is_current_stream_capturing()):
+            self._insert(name, tuple(weights), buffer, None, pack)
+
     def refresh(self) -> int:
         """Pack every live entry again from its weights' current values, into its own
         buffers, on the current stream, and record the new versions.  For graphs captured
@@ -410,26 +470,38 @@ class PackCache:
         addresses).  Returns the number of entries repacked."""
         n = 0
         with self._lock:
-            for entry in list(self._entries.values()):
+            for entry in [e for c in (self, *self._children) for e in c._entries.values()]:
                 keys = [r() for r in entry.refs]
                 if any(k is None for k in keys) or entry.spec is None:
                     continue
-                dt, d, h, e, s = entry.spec
-                ws = [k if k.dtype == dt else k.detach().to(dt) for k in keys]
-                ws = [w.contiguous() for w in ws]
-                a = nat.ExpertsArgs(dtype=_DT[dt], activation=0, n_tokens=0, d_model=d,
-                                    d_hidden=h, n_experts=e, n_shared=s, top_k=1,
-                                    reserved0=0, l_cap=0, w_in=ws[0].data_ptr(),
-                                    w_out=ws[1].data_ptr(),
-                                    w_sh_in=ws[2].data_ptr() if s else None,
-                                    w_sh_out=ws[3].data_ptr() if s else None)
-                nat.check(nat.lib().nsmoe_pack_weights(a, entry.p_in.data_ptr(),
-                                                       entry.p_out.data_ptr(), _stream()),
-                          "nsmoe_pack_weights")
+                if callable(entry.spec):
+                    entry.spec(keys, entry.p_in)
+                else:
+                    _pack_experts(entry.spec, keys, entry.p_in, entry.p_out)
                 entry.states = tuple(self._state(k) for k in keys)
-                entry.packed_on(torch.cuda.current_stream(entry.p_in.device))
+                if entry.p_in.is_cuda:
+                    entry.packed_on(torch.cuda.current_stream(entry.p_in.device))
                 n += 1
         return n
+
+
+def _pack_experts(spec, weights, p_in: Tensor, p_out: Tensor) -> None:
+    """The expert weights of `spec` into existing buffers, on the current stream."""
+    dt, d, h, e, s = spec
+    ws = [w if w.dtype == dt else w.detach().to(dt) for w in weights]
+    ws = [w.contiguous() for w in ws]
+    a = nat.ExpertsArgs(dtype=_DT[dt], activation=0, n_tokens=0, d_model=d,
+                        d_hidden=h, n_experts=e, n_shared=s, top_k=1,
+                        reserved0=0, l_cap=0, w_in=ws[0].data_ptr(),
+                        w_out=ws[1].data_ptr(),
+                        w_sh_in=ws[2].data_ptr() if s else None,
+                        w_sh_out=ws[3].data_ptr() if s else None)
+    nat.check(nat.lib().nsmoe_pack_weights(a, p_in.data_ptr(), p_out.data_ptr(), _stream()),
+              "nsmoe_pack_weights")
+
+
+def _empty_pack_cache(capacity: int, is_child: bool) -> PackCache:
+    return PACKS.child(capacity) if is_child else PackCache(capacity)
 
 
 PACKS = PackCache()

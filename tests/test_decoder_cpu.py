@@ -177,3 +177,65 @@ def test_plain_attention_reads_the_current_output_weight(monkeypatch):
             assert torch.equal(att(z), o.view(2, 3, 64) @ att.W_O)
             att.W_O.data.add_(1.0)
             att.W_O = torch.nn.Parameter(att.W_O.data)
+
+
+def _unpacked(w):
+    return w.permute(1, 2, 4, 0, 3).reshape(w.shape[1] * 32, w.shape[0] * 16)
+
+
+def test_projection_packs_follow_their_parameters():
+    """A kept pack belongs to the parameter objects: it is reused while they are unchanged,
+    and made anew after an in-place update, and for another parameter at the same address and
+    version.  After a write through `.data` PACKS.clear() drops it and PACKS.refresh() rewrites
+    it in its place."""
+    from nanospeaker_amd.moe_kernel import PACKS
+
+    att, dt = _small_attention(), torch.float32
+    packed = lambda: att._packed("o", dt, att.W_O)
+    first = packed()
+    assert torch.equal(_unpacked(first), att.W_O)
+    assert packed() is first
+    with torch.no_grad():
+        att.W_O.mul_(2.0)
+    second = packed()
+    assert torch.equal(_unpacked(second), att.W_O) and not torch.equal(first, second)
+    att.W_O.data.add_(1.0)
+    att.W_O = torch.nn.Parameter(att.W_O.data)
+    third = packed()
+    assert torch.equal(_unpacked(third), att.W_O)
+    att.W_O.data.add_(1.0)
+    PACKS.clear()
+    assert torch.equal(_unpacked(packed()), att.W_O)
+    with torch.inference_mode():
+        PACKS.clear()
+        kept = packed()
+    qkv = att._packed("qkv", torch.bfloat16, att.W_q, att.W_k, att.W_v)
+    att.W_O.data.add_(1.0)
+    att.W_k.data.add_(1.0)
+    assert PACKS.refresh() >= 2
+    assert packed() is kept and torch.equal(_unpacked(kept), att.W_O)
+    assert torch.equal(_unpacked(qkv),
+                       torch.cat((att.W_q, att.W_k, att.W_v), dim=1).to(torch.bfloat16))
+
+
+def test_projection_packs_stay_with_their_module():
+    """A deep copy or a pickled module starts with no packs and then keeps its own; a module
+    that kept them in a dict before works on."""
+    import copy
+    import pickle
+
+    from nanospeaker_amd.moe_kernel import PACKS
+
+    att = _small_attention()
+    att._packed("o", torch.float32, att.W_O)
+    for other in (copy.deepcopy(att), pickle.loads(pickle.dumps(att))):
+        assert len(other._packs) == 0 and len(att._packs) == 1
+        with torch.no_grad():
+            other.W_O.neg_()
+        assert torch.equal(_unpacked(other._packed("o", torch.float32, other.W_O)), other.W_O)
+        assert other._packs in PACKS._children
+        PACKS.clear()
+        assert len(other._packs) == 0
+        att._packed("o", torch.float32, att.W_O)
+    att._packs = {"o": ((), att.W_O.detach())}
+    assert torch.equal(_unpacked(att._packed("o", torch.float32, att.W_O)), att.W_O)

@@ -14,6 +14,7 @@ pytest.importorskip("nanospeaker_amd.moe_kernel")
 from nanospeaker_amd import _native as nat  # noqa: E402
 from nanospeaker_amd.decoder import (Attention, DecoderConfig, Rotary, linear,  # noqa: E402
                                      pack_linear)
+from nanospeaker_amd.moe_kernel import PACKS  # noqa: E402
 
 DEV = "cuda"
 
@@ -116,3 +117,88 @@ def test_plain_attention_reads_the_current_output_weight():
             o = att._kernel_attention(z).view(2, 70, -1)
             assert torch.equal(att(z), o @ att.W_O)
             att.W_O.data.mul_(2.0)
+
+
+def _attention_and_inputs(rotary=None):
+    cfg = DecoderConfig()
+    att = Attention(cfg, rotary or Rotary(64, cfg.rope_base), None).to(DEV, torch.bfloat16).eval()
+    g = torch.Generator().manual_seed(3)
+    x, z = (torch.randn(2, 70, 576, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+    return att, x, z
+
+
+def test_projection_packs_on_another_stream():
+    """A pack made behind long work on one stream is waited for by a call on another one."""
+    att, x, z = _attention_and_inputs()
+    with torch.no_grad():
+        ref = att.forward_residual(x, z)
+        PACKS.clear()
+        torch.cuda.synchronize()
+        one, two = torch.cuda.Stream(), torch.cuda.Stream()
+        with torch.cuda.stream(one):
+            torch.cuda._sleep(20_000_000)
+            first = att.forward_residual(x, z)
+        with torch.cuda.stream(two):
+            second = att.forward_residual(x, z)
+        torch.cuda.synchronize()
+        assert torch.equal(first, ref) and torch.equal(second, ref)
+
+
+def _capture(fn):
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = fn()
+    return graph, out
+
+
+@pytest.mark.parametrize("warm", [True, False])
+def test_captured_projections_follow_the_weights(warm):
+    """A captured sublayer packs in its graph, whether its weights' packs were kept before or
+    not: every replay has the weights of that moment, and eager calls after a capture (with no
+    replay yet) and between replays have theirs."""
+    att, x, z = _attention_and_inputs()
+    other, _, _ = _attention_and_inputs(att.rotary)
+    with torch.no_grad():
+        other.forward_residual(x, z)  # the rotary tables
+        if warm:
+            att.forward_residual(x, z)
+        graph, out = _capture(lambda: att.forward_residual(x, z))
+        for step in range(4):
+            eager = att.forward_residual(x, z)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager), step
+            for w in (att.W_O, att.W_k):
+                w.mul_(1.5)
+
+
+def test_captured_projections_share_kept_packs():
+    """With share_with_graphs a capture reads the kept packs, which stay until clear(): a
+    replay has the new weights after refresh(), also when the layer object itself is gone."""
+    att, x, z = _attention_and_inputs()
+    weights = (att.W_q, att.W_k, att.W_v, att.W_O)
+    gains_and_tables = (att.q_norm, att.k_norm, att.rotary)
+    with torch.no_grad():
+        att.forward_residual(x, z)
+        PACKS.share_with_graphs = True
+        try:
+            graph, out = _capture(lambda: att.forward_residual(x, z))
+        finally:
+            PACKS.share_with_graphs = False
+        for step in range(3):
+            ref = att.forward_residual(x, z)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, ref), step
+            for w in weights:
+                w.mul_(1.25)
+            assert PACKS.refresh() >= 2
+        ref = att.forward_residual(x, z)
+        del att
+        spare = [torch.full((576 * 960,), float("nan"), device=DEV, dtype=torch.bfloat16)
+                 for _ in range(8)]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and len(spare) == 8 and gains_and_tables
+    PACKS.clear()
