@@ -595,8 +595,11 @@ __global__ void __launch_bounds__(NT, DT == DT_F32 ? 3 : 1) expert_bwd_kernel(Ex
 // index in memory, so both operands are staged transposed (TransStage) into swizzled
 // LDS: KCH chunks of 32 rows per barrier, the A and B chunks of a stage staged by
 // disjoint thread ranges so every wave shares the transposes.  The row -> token lookups
-// of the work item's rows are read once into LDS.  Tile BMo x BNo =
-// (WGM * TM * 16) x (WGN * TN * 16).
+// of the work item's rows are read into LDS a window at a time: 3 KB beside the 48 KB of the
+// 16-bit types' stages leave room for three workgroups per CU, which a table for the longest
+// chunk (32 KB) does not (training step, d 572, H 124, top-6 of 76 + 2, T = 8192, bf16: 1728 us
+// with that table, 1328 so).  Tile BMo x BNo = (WGM * TM * 16) x (WGN * TN * 16).
+constexpr int DW_TOK_ROWS = 768;
 
 template <int MODE> struct DwShape;
 template <> struct DwShape<0> {  // dW_in: 64 x 128 tiles, waves side by side along N
@@ -708,7 +711,7 @@ __global__ void __launch_bounds__(NT) dw_kernel(ExpParams p) {
   constexpr int TA = Stager::TA, TB = Stager::TB;
   constexpr int STAGE = KCH * (TA + TB);
   __shared__ __attribute__((aligned(16))) char s_stage[2][STAGE];
-  __shared__ int s_tok[DW_RC_MAX];
+  __shared__ int s_tok[DW_TOK_ROWS];
   __shared__ int s_loc[3];
 
   const int d = p.d, H = p.H, twoH = 2 * p.H;
@@ -739,21 +742,27 @@ __global__ void __launch_bounds__(NT) dw_kernel(ExpParams p) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lc = lane & 15, lg = lane >> 4;
   const int wm = wave / S::WGN, wn = wave % S::WGN;
 
-  for (int r = r0 + tid; r < r1; r += NT)
-    s_tok[r - r0] = g < p.E ? p.sorted_ids[rs + r] / p.k : r;
-  __syncthreads();
+  // The tokens of rows [w0, w0 + DW_TOK_ROWS) of the chunk.
+  int w0 = r0;
+  auto window = [&](int from) {
+    w0 = from;
+    for (int r = from + tid; r < min(r1, from + DW_TOK_ROWS); r += NT)
+      s_tok[r - from] = g < p.E ? p.sorted_ids[rs + r] / p.k : r;
+    __syncthreads();
+  };
+  window(r0);
 
   const T* X = (const T*)p.x;
   const T* DA = (const T*)p.da1;
   const T* HB = (const T*)p.hbuf;
   const T* DO = (const T*)p.dout;
   auto rowA = [&](int r) -> const T* {
-    if (MODE == 0) return X + (int64_t)s_tok[r - r0] * d;
+    if (MODE == 0) return X + (int64_t)s_tok[r - w0] * d;
     return HB + (rs + r) * H;
   };
   auto rowB = [&](int r) -> const T* {
     if (MODE == 0) return DA + (rs + r) * twoH;
-    return DO + (int64_t)s_tok[r - r0] * d;
+    return DO + (int64_t)s_tok[r - w0] * d;
   };
 
   Stager stg;
@@ -764,7 +773,8 @@ __global__ void __launch_bounds__(NT) dw_kernel(ExpParams p) {
   for (int i = 0; i < S::TM; ++i)
 #pragma unroll
     for (int j = 0; j < S::TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int KS = KCH * G::KC;
+  constexpr int KS = KCH * G::KC;
+  static_assert(DW_TOK_ROWS % KS == 0, "windows of whole steps");
   const int ns = (r1 - r0 + KS - 1) / KS;
   if (ns > 0) {
     load(r0);
@@ -773,7 +783,12 @@ __global__ void __launch_bounds__(NT) dw_kernel(ExpParams p) {
     for (int st = 0; st < ns; ++st) {
       const int cur = st & 1;
       const bool more = st + 1 < ns;
-      if (more) load(r0 + (st + 1) * KS);
+      if (more) {
+        const int k0 = r0 + (st + 1) * KS;
+        // The barrier that ended the last step is behind every read of the window before.
+        if (k0 - w0 == DW_TOK_ROWS) window(k0);
+        load(k0);
+      }
 #pragma unroll
       for (int q = 0; q < KCH; ++q) {
         const char* ta = s_stage[cur] + q * TA;

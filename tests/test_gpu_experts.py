@@ -241,3 +241,23 @@ def test_forward_is_deterministic():
     assert torch.equal(a, b)
     for n in ga:
         assert torch.equal(ga[n], gb[n]), n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T", [13824, 14000, 28000])
+def test_general_dw_kernel_token_windows(T, dtype):
+    """Shapes off the vector path (d % 8 != 0) run dw_kernel, which reads the tokens of a
+    chunk's rows a window of 768 at a time: the shared expert's chunks of 768 rows (one
+    window), 800 and 1568 (two and three).  The routed rows' tokens are not their numbers."""
+    d, E, H = 1156, 3, 12
+    p = R.make_params(5, d, E, 18, n_shared=1).to(dtype=dtype)
+    assert p.W_out.shape == (E, H, d)
+    g = torch.Generator().manual_seed(T)
+    x, gout = (torch.randn(T, d, generator=g).to(dtype) for _ in range(2))
+    ti = (torch.arange(T) % 3 != 0).long()[:, None]
+    tw = torch.rand(T, 1, generator=g).to(dtype)
+    ref_out, ref_g = oracle_fwd_bwd(p, x, gout, tw, ti, "silu")
+    out, grads = gpu_fwd_bwd(p, x, gout, tw, ti, "silu")
+    check("out", out, ref_out, dtype)
+    for n in ref_g:
+        check(f"grad {n}", grads[n], ref_g[n], dtype)

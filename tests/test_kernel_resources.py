@@ -1,0 +1,65 @@
+"""
+What the built kernels take of a compute unit, read from the metadata of libnsmoe.so's own
+code objects (the LDS and register figures that the compiler writes beside each kernel).
+The launch rules count on these workgroups per CU; a larger table or tile lowers them
+without a word.
+"""
+
+import re
+import shutil
+import struct
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from nanospeaker_amd import _native as nat
+
+LDS_PER_CU = 160 * 1024
+READELF = shutil.which("llvm-readelf") or "/opt/rocm/llvm/bin/llvm-readelf"
+OBJCOPY = shutil.which("llvm-objcopy") or "/opt/rocm/llvm/bin/llvm-objcopy"
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{mangled name: {"lds": bytes, "vgprs": n, "spills": n}} of every kernel."""
+    if not (Path(READELF).exists() and Path(OBJCOPY).exists() and nat.LIB_PATH.exists()):
+        pytest.skip("needs the LLVM binutils and the built library")
+    tmp = tmp_path_factory.mktemp("code_objects")
+    fat = tmp / "fatbin"
+    subprocess.run([OBJCOPY, f"--dump-section=.hip_fatbin={fat}", str(nat.LIB_PATH), "/dev/null"],
+                   check=True)
+    blob, out = fat.read_bytes(), {}
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    for at in (m.start() for m in re.finditer(magic, blob)):
+        n, pos = struct.unpack_from("<Q", blob, at + len(magic))[0], at + len(magic) + 8
+        for _ in range(n):
+            off, size, length = struct.unpack_from("<QQQ", blob, pos)
+            triple = blob[pos + 24:pos + 24 + length].decode()
+            pos += 24 + length
+            if "gfx950" not in triple or not size:
+                continue
+            obj = tmp / "object.elf"
+            obj.write_bytes(blob[at + off:at + off + size])
+            notes = subprocess.run([READELF, "--notes", str(obj)], check=True,
+                                   capture_output=True, text=True).stdout
+            for part in notes.split("- .agpr_count:")[1:]:
+                field = lambda key: re.search(rf"\.{key}:\s+(\S+)", part).group(1)
+                name = re.search(r"^    \.name:\s+(\S+)", part, re.M).group(1)
+                out[name] = {"lds": int(field("group_segment_fixed_size")),
+                             "vgprs": int(field("vgpr_count")),
+                             "spills": int(field("vgpr_spill_count"))}
+    assert len(out) > 100
+    return out
+
+
+def _of(kernels, pattern):
+    found = {n: k for n, k in kernels.items() if re.search(pattern, n)}
+    assert found, pattern
+    return found
+
+
+def test_general_dw_kernel_fits_three_times_in_a_cu(kernels):
+    """dw_kernel in 16-bit types (DT 0 and 1, both modes)."""
+    for name, k in _of(kernels, r"dw_kernelILi[01]ELi[01]E").items():
+        assert 3 * k["lds"] <= LDS_PER_CU, (name, k)
