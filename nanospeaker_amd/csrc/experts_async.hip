@@ -14,6 +14,7 @@
 // register-staged kernels.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -1824,6 +1825,7 @@ template <> struct DwTile<1> {  // dW_out [H, d]: 128 x 192 tiles
 template <int DT>
 constexpr int dw_step_rows() { return 64 / Geo<DT>::ES; }
 
+// (The tokens of a chunk's rows are a table in dynamic LDS, as long as the call's chunks.)
 template <int DT, int S>
 struct DwLds {
   static constexpr int STAGE =
@@ -1831,7 +1833,6 @@ struct DwLds {
   static_assert(STAGE == dw_step_rows<DT>() * (DwTile<1>::BMT + DwTile<1>::BNT) * Geo<DT>::ES,
                 "both modes stage the same bytes per step");
   char ring[S][STAGE];
-  int tok[DW_RC_MAX];
   int loc[3];
 };
 
@@ -1859,7 +1860,7 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
   constexpr int LOADS = NBLK / 4;
   static_assert(STAGE == DwLds<DT, S>::STAGE, "stage layout");
   auto& s_ring = L.ring;
-  int* s_tok = L.tok;
+  extern __shared__ int s_tok[];  // [p.dw_rc]
   int* s_loc = L.loc;
 
   const int d = p.d, H = p.H, twoH = 2 * p.H;
@@ -2105,17 +2106,22 @@ int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_ou
     gr.end[i] = (int)end;
   }
   if (end <= 0) return NSMOE_OK;
-  // Ring stages: 2 (one step of copies in flight, two workgroups per CU), which
-  // measured ~1% faster per training step than 3; the "dw_stages" option asks for 3 or 4.
+  // Ring stages: 2 (one step of copies in flight); the "dw_stages" option asks for 3 or 4.
+  // A stage is 20 KB and the token table 4 bytes a row of a chunk: two workgroups per CU at 2
+  // stages, at 3 while a chunk has at most 5,100 rows, one at 4.  (fp32 at 2 stages would fit
+  // three; two, kept by its table's least size, are 2 % of the training step faster: d 576,
+  // H 128, top-6 of 76 + 2, T = 2048 510 us against 520, T = 8192 1409 against 1430.)
+  // Training step in bf16, T = 8192: 283 us at 2 stages, 283 at 3, 314 at 4.
   const int st = option(OPT_DW_STAGES) ? (int)option(OPT_DW_STAGES) : 2;
   KernelTimer timer("dw", s);
   const unsigned grid = (unsigned)end;
+  const size_t tok = std::max<size_t>((size_t)q_in.dw_rc * sizeof(int), dtype == DT_F32 ? 14336 : 0);
   auto go = [&](auto dt_tag) {
     constexpr int DT = decltype(dt_tag)::value;
-    if constexpr (DT == DT_F32) dw_pair_kernel<DT, 2><<<grid, NT, 0, s>>>(q_in, q_out, gr);
-    else if (st == 3) dw_pair_kernel<DT, 3><<<grid, NT, 0, s>>>(q_in, q_out, gr);
-    else if (st == 4) dw_pair_kernel<DT, 4><<<grid, NT, 0, s>>>(q_in, q_out, gr);
-    else dw_pair_kernel<DT, 2><<<grid, NT, 0, s>>>(q_in, q_out, gr);
+    if constexpr (DT == DT_F32) dw_pair_kernel<DT, 2><<<grid, NT, tok, s>>>(q_in, q_out, gr);
+    else if (st == 3) dw_pair_kernel<DT, 3><<<grid, NT, tok, s>>>(q_in, q_out, gr);
+    else if (st == 4) dw_pair_kernel<DT, 4><<<grid, NT, tok, s>>>(q_in, q_out, gr);
+    else dw_pair_kernel<DT, 2><<<grid, NT, tok, s>>>(q_in, q_out, gr);
   };
   if (dtype == DT_BF16) go(std::integral_constant<int, DT_BF16>{});
   else if (dtype == DT_F16) go(std::integral_constant<int, DT_F16>{});

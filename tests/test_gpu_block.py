@@ -264,6 +264,17 @@ def test_dw_chunk_edges(T, dtype):
     run_case(T, train=True, backward=True, d=128, E=8, d_ff=96, k=4, S=1, dtype=dtype)
 
 
+@pytest.mark.parametrize("stages", [2, 3, 4])
+@pytest.mark.parametrize("T", [1, 513, 2500])
+def test_dw_ring_stages(stages, T):
+    """The dW kernel's ring at each number of stages, its token table behind it, with chunks
+    shorter than the ring, of one step more than 512 rows' and of several hundred rows."""
+    from tests.helpers import lib_options
+
+    with lib_options(dw_stages=stages):
+        run_case(T, train=True, backward=True, d=128, E=8, d_ff=96, k=4, S=1)
+
+
 @pytest.mark.parametrize("T", [15, 63, 65, 400])
 @pytest.mark.parametrize("cfg", [dict(), dict(d=320, E=12, k=3, S=1, d_ff=192),
                                  dict(d=384, E=10, k=2, S=0, d_ff=144), dict(d=128, E=6, k=2, S=2,

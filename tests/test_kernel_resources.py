@@ -63,3 +63,12 @@ def test_general_dw_kernel_fits_three_times_in_a_cu(kernels):
     """dw_kernel in 16-bit types (DT 0 and 1, both modes)."""
     for name, k in _of(kernels, r"dw_kernelILi[01]ELi[01]E").items():
         assert 3 * k["lds"] <= LDS_PER_CU, (name, k)
+
+
+def test_dw_pair_kernel_fits_twice_in_a_cu(kernels):
+    """dw_pair_kernel at two stages in every type, and at three in 16-bit types: two
+    workgroups beside their token tables of 4 bytes a row, for the longest chunks (8192 rows)
+    at two stages and chunks of 5000 rows (184 k rows of work) at three."""
+    for pattern, rows in ((r"dw_pair_kernelILi[012]ELi2E", 8192), (r"dw_pair_kernelILi[01]ELi3E", 5000)):
+        for name, k in _of(kernels, pattern).items():
+            assert 2 * (k["lds"] + 4 * rows) <= LDS_PER_CU, (name, k)
