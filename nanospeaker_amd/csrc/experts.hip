@@ -836,21 +836,35 @@ __global__ void __launch_bounds__(NT) dw_reduce_kernel(DwReduceArgs r) {
   dw_reduce_wg<DT>(r, blockIdx.x);
 }
 
-// Rows per dW chunk: a thirty-sixth of all rows, a multiple of 32.  A chunk longer than that
-// is an item that outlasts the launch's other work; a shorter one splits more groups, and
-// every chunk of a split group writes an fp32 partial of 885 KB (d 576, H 128) that the
-// reduce reads again.  Measured training steps (us; 76 + 2 experts, top-6; rows in brackets)
-// by chunk length, balanced routing unless noted:
+// Rows per dW chunk: a thirty-sixth of all rows, or less where a chunk has few output tiles, so
+// that the launch has items (chunks x tiles) for the chip's workgroup slots: 324 on the ring
+// kernel (two slots a CU), 1152 on the general one (three, and shorter items); a multiple
+// of 32.  A chunk longer than that is an item that outlasts the launch's other work; a shorter
+// one splits more groups, and every chunk of a split group writes an fp32 partial of 885 KB (d
+// 576, H 128) that the reduce reads again.  Measured training steps by chunk length (us; bf16,
+// top-6 of 76 + 2, d 576, H 128, 9 tiles, balanced routing unless noted; rows in brackets):
 //   T 2047 (16 k)           512: 159   768: 159   1536: 166   3072: 173
 //   T 8192 (66 k)           768: 287   1536: 281  2048: 279   3072: 293
 //   T 16384 (131 k)         768: 649   1536: 495  2048: 492   3072: 492   8192: 548
 //   T 16384, Zipf           1536: 534  3072: 528  8192: 583
 // (768 at T 16384 cuts every routed group in two: 134 MB of partials written and read.)
-// Below 512 rows a chunk is a few k-steps and the item's own setup dominates; 8192 is what
-// the items' token table in LDS holds.
+// Few tiles (top-2 of 8 + 1, or of 4 + 1 for d 64), a thirty-sixth of the rows last:
+//   d 64, H 32, 2 tiles, T 131072 (393 k)   768: 396  1024: 392  2048: 386  4096: 417   8192: 479
+//   d 128, H 64, 2, T 65536 (197 k)         768: 288  1024: 276  2048: 285  4096: 313   5472: 333
+//   d 256, H 64, 4, T 65536 (197 k)         768: 411  1024: 402  2048: 393  4096: 432   5472: 456
+// General kernel (H 60 in fp16, H 124 with top-6 of 76 + 2):
+//   d 300, H 60, 10 tiles, T 32768 (98 k)   512: 791  768: 746   1536: 860  2752: 1021
+//   d 572, H 124, 27, T 8192 (66 k)         512: 1362 768: 1328  1536: 1303 1824: 1328  2048: 1346
+// Below 512 rows a chunk is a few k-steps and the item's own setup dominates; a chunk of 8192
+// rows has a token table of 32 KB in the ring kernel's LDS.  The rule goes by the shape alone
+// (not the pointers' alignment or the device), as the workspace is sized by it beforehand.
 static int64_t dw_rows_per_chunk(const nsmoe_experts_args* a) {
-  const int64_t rows = a->n_tokens * (a->top_k + a->n_shared);
-  return std::clamp<int64_t>(cdiv(rows, 36 * 32) * 32, DW_RC_MIN, DW_RC_MAX);
+  const int64_t d = a->d_model, H = a->d_hidden, rows = a->n_tokens * (a->top_k + a->n_shared);
+  const bool ring = d % 8 == 0 && H % 8 == 0;
+  const int64_t tiles = ring ? dw_pair_tiles((int)d, (int)H)
+                             : cdiv(d, 64) * cdiv(2 * H, 128) + cdiv(H, 128) * cdiv(d, 64);
+  const int64_t chunks = std::max<int64_t>(36, cdiv(ring ? 324 : 1152, tiles));
+  return std::clamp<int64_t>(cdiv(rows, chunks * 32) * 32, DW_RC_MIN, DW_RC_MAX);
 }
 
 // Workgroups of the dW reduce: one per (group, mode, block) item of the shared groups and of

@@ -2062,11 +2062,12 @@ __device__ __forceinline__ void dw_item(const ExpParams& p, bool shared, int ite
 // Output tiles per (group, row chunk) of a dW mode: the run of items that read the same
 // token rows, dealt to one XCD together.
 template <int MODE>
-__device__ __forceinline__ int dw_run(const ExpParams& p) {
+__host__ __device__ __forceinline__ int dw_run(int d, int H) {
   using Tl = DwTile<MODE>;
-  const int Md = MODE == 0 ? p.d : p.H, Nd = MODE == 0 ? 2 * p.H : p.d;
+  const int Md = MODE == 0 ? d : H, Nd = MODE == 0 ? 2 * H : d;
   return ((Md + Tl::BMT - 1) / Tl::BMT) * ((Nd + Tl::BNT - 1) / Tl::BNT);
 }
+int dw_pair_tiles(int d, int H) { return dw_run<0>(d, H) + dw_run<1>(d, H); }
 
 // dW_in and dW_out items in one launch, in four parts, each dealt over the XCDs on its own
 // (every part is a multiple of 8 blocks, so a part's block b sits on XCD b % 8): the shared
@@ -2084,8 +2085,8 @@ __global__ void __launch_bounds__(NT, 2) dw_pair_kernel(ExpParams p_in, ExpParam
   const int b = blockIdx.x;
   const int part = (b >= gr.end[0]) + (b >= gr.end[1]) + (b >= gr.end[2]);
   const int b0 = part ? gr.end[part - 1] : 0, n = gr.end[part] - b0;
-  if (part & 1) dw_item<DT, 1, S>(p_out, part < 2, xcd_deal(b - b0, n, dw_run<1>(p_out)), lds);
-  else dw_item<DT, 0, S>(p_in, part < 2, xcd_deal(b - b0, n, dw_run<0>(p_in)), lds);
+  if (part & 1) dw_item<DT, 1, S>(p_out, part < 2, xcd_deal(b - b0, n, dw_run<1>(p_out.d, p_out.H)), lds);
+  else dw_item<DT, 0, S>(p_in, part < 2, xcd_deal(b - b0, n, dw_run<0>(p_in.d, p_in.H)), lds);
 }
 
 int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_out,
@@ -2094,8 +2095,7 @@ int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_ou
   if (q_in.T * q_in.d >= (int64_t(1) << 31)) return -1;  // token offsets are int32
   const int d = q_in.d, H = q_in.H;
   const int64_t shared_chunks = (int64_t)q_in.S * dw_chunks((int)q_in.T, q_in.dw_rc);
-  const int64_t t_in = cdiv(d, DwTile<0>::BMT) * cdiv(2 * H, DwTile<0>::BNT);
-  const int64_t t_out = cdiv(H, DwTile<1>::BMT) * cdiv(d, DwTile<1>::BNT);
+  const int64_t t_in = dw_run<0>(d, H), t_out = dw_run<1>(d, H);
   DwGrid gr;
   int64_t end = 0;
   const int64_t items[4] = {shared_chunks * t_in, shared_chunks * t_out, routed_chunks * t_in,

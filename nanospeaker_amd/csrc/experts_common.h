@@ -164,6 +164,8 @@ int launch_fwd_async(int dtype, const ExpParams& p, int nbw, int64_t grid, hipSt
 // tiles to scan the expert ids (p.topk_idx set).
 bool fwd_scan_shape(int dtype, const ExpParams& p, int nbw);
 constexpr int SCAN_MAX_PAIRS = 2048;  // 8 ids a lane
+// Output tiles of both dW modes per row chunk in launch_dw_pair_async.
+int dw_pair_tiles(int d, int H);
 // Both dW modes in one launch (q_in: dW_in, q_out: dW_out pointers and partials).
 int launch_dw_pair_async(int dtype, const ExpParams& q_in, const ExpParams& q_out,
                          int64_t routed_chunks, hipStream_t s);

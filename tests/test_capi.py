@@ -131,6 +131,35 @@ def test_workspace_sizes_are_positive_and_grow():
     assert nat.lib().nsmoe_dispatch_workspace_size(49152, 1000) == 192 * 1000 * 4
 
 
+def dw_rows_per_chunk(d, H, T, k, S):
+    """The row chunks of the dW work: at least 36, and more where few output tiles (192 x 128
+    and 128 x 192 on the ring kernel, 64 x 128 and 128 x 64 off the vector path) would leave
+    the launch short of items; 512 to 8192 rows each, whole 32s."""
+    up = lambda a, b: -(-a // b)
+    if d % 8 == 0 and H % 8 == 0:
+        tiles, items = up(d, 192) * up(2 * H, 128) + up(H, 128) * up(d, 192), 324
+    else:
+        tiles, items = up(d, 64) * up(2 * H, 128) + up(H, 128) * up(d, 64), 1152
+    rc = up(T * (k + S), max(36, up(items, tiles)) * 32) * 32
+    return min(max(rc, 512), 8192)
+
+
+@pytest.mark.parametrize("d,H,E,k,S,T", [
+    (576, 128, 76, 6, 2, 8192), (576, 128, 76, 6, 2, 100), (64, 32, 4, 2, 1, 131072),
+    (128, 64, 8, 2, 1, 65536), (256, 64, 8, 2, 1, 65536), (2048, 512, 8, 2, 1, 65536),
+    (300, 60, 8, 2, 1, 32768), (572, 124, 76, 6, 2, 8192), (100, 36, 16, 2, 0, 500_000)])
+def test_dw_chunks_by_shape(d, H, E, k, S, T):
+    """The backward's workspace holds the partials of the chunks that the shape's rule gives."""
+    a = nat.ExpertsArgs(dtype=0, activation=0, n_tokens=T, d_model=d, d_hidden=H, n_experts=E,
+                        n_shared=S, top_k=k, l_cap=mk._l_cap(T * k, E))
+    al = lambda n: -(-n // 256) * 256
+    rows, rc = a.l_cap + S * T, dw_rows_per_chunk(d, H, T, k, S)
+    partials = 2 * -(-T * k // rc) + 1 + S * -(-T // rc)
+    want = sum(al(rows * n * 2) for n in (2 * H, H, d)) + al(partials * d * 2 * H * 4) + al(
+        partials * H * d * 4)
+    assert nat.lib().nsmoe_experts_bwd_workspace_size(a) == want
+
+
 def test_pack_sizes_match_the_fragment_layout():
     a = nat.ExpertsArgs(dtype=0, activation=0, n_tokens=8192, d_model=576, d_hidden=128,
                         n_experts=76, n_shared=2, top_k=6, l_cap=mk._l_cap(49152, 76))
