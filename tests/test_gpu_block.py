@@ -264,6 +264,13 @@ def test_dw_chunk_edges(T, dtype):
     run_case(T, train=True, backward=True, d=128, E=8, d_ff=96, k=4, S=1, dtype=dtype)
 
 
+def test_dw_reduce_of_many_split_groups():
+    """40 routed groups and the shared one, nearly all of several chunks, with 24 blocks of
+    dW elements a group: more items than the reduce has workgroups, so each takes several."""
+    ref = run_case(8192, train=True, backward=True, d=128, E=40, d_ff=96, k=4, S=1)
+    assert int((ref.counts > 512).sum()) * 24 > 768
+
+
 @pytest.mark.parametrize("stages", [2, 3, 4])
 @pytest.mark.parametrize("T", [1, 513, 2500])
 def test_dw_ring_stages(stages, T):
