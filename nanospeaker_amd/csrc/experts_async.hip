@@ -2137,10 +2137,17 @@ static int64_t tile_grid(const ExpParams& p, int bm) {
   return cdiv(M, bm) + nonempty + (int64_t)p.S * cdiv(p.T, bm);
 }
 
+// Scanning tiles: (E + S) ceil(T / 32) workgroups, each of which reads all the ids, most of
+// them to find no rows once T / 32 exceeds a group's tiles.  Up to twelve a CU: a captured call
+// (d 576, 76 + 2 experts, top-1; us, scanning / with a dispatch) takes 40.1 / 44.6 at T = 512 (1248
+// workgroups), 43.3 / 46.3 at 1024 (2496), 47.9 / 46.2 at 1536 (3744), 53.9 / 46.9 at 2048
+// (4992).  Top-6 stays under 900.
+static int64_t scan_grid(const ExpParams& p) { return (p.E + p.S) * cdiv(p.T, 32); }
+
 template <int DT, int NBW>
 static void fwd_reg_launch(const ExpParams& p, int mb, int dist, hipStream_t s) {
   if (p.topk_idx) {  // fwd_scan_shape
-    const unsigned gs = (unsigned)((p.E + p.S) * cdiv(p.T, 32));
+    const unsigned gs = (unsigned)scan_grid(p);
     if (dist == 6) expert_fwd_reg_kernel<DT, NBW, 2, 6, true><<<gs, NT, 0, s>>>(p);
     else expert_fwd_reg_kernel<DT, NBW, 2, 2, true><<<gs, NT, 0, s>>>(p);
     return;
@@ -2179,7 +2186,8 @@ static bool fwd_reg_shape(const ExpParams& p) {
 
 bool fwd_scan_shape(int dtype, const ExpParams& p, int nbw) {
   return p.fast && nbw <= 2 && (dtype == DT_BF16 || dtype == DT_F16) && fwd_reg_shape(p) &&
-         p.T * p.k <= SCAN_MAX_PAIRS && fwd_row_blocks(p) == 2;
+         p.T * p.k <= SCAN_MAX_PAIRS && scan_grid(p) <= 12 * (int64_t)device_cus() &&
+         fwd_row_blocks(p) == 2;
 }
 
 int launch_fwd_async(int dtype, const ExpParams& p, int nbw, int64_t grid, hipStream_t s) {

@@ -329,6 +329,25 @@ def test_decode_without_dispatch_matches_the_dispatched_forward(T, collapsed):
                 assert n1 - n0 == (3 if 6 * T <= 2048 else 4), (T, n1 - n0)
 
 
+@pytest.mark.parametrize("T,k,scans", [(1024, 1, True), (1536, 1, False), (2048, 1, False),
+                                       (341, 6, True), (342, 6, False), (1024, 2, True)])
+def test_scanning_tiles_stop_where_a_dispatch_is_cheaper(T, k, scans):
+    """Calls without gradients go without the dispatch launch while their scanning tiles are
+    at most twelve a CU: three launches, against four.  (76 + 2 experts on 256 CUs: 3072
+    workgroups, T up to 1248 at top-1, where the pairs alone would allow 2048.)"""
+    from nanospeaker_amd import _native as nat
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes stand for 256 CUs")
+    m, _, x, _ = build(T, k=k)
+    m, x = m.to(DEV).eval(), x.to(DEV)
+    with torch.no_grad():
+        m(x)  # the packs
+        n0 = nat.launch_count()
+        m(x)
+    assert nat.launch_count() - n0 == (3 if scans else 4)
+
+
 @pytest.mark.parametrize("T", [1, 15, 17, 31, 33, 49])
 def test_fp32_tile_edges(T):
     """fp32's 32-row tiles: groups of every remainder of a tile (the shared groups hold all T
