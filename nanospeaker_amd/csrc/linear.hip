@@ -5,9 +5,9 @@
 //
 // What bounds it: at K = 576 a tile's operands are used for few MFMAs, so a kernel that
 // stages both operands per k-step waits on its copies (the library's 256 x 256 kernels ran
-// these two shapes at 566 and 410 TFLOP/s).  Here a workgroup of 12 waves keeps its 128 rows of
-// x whole in LDS (147 KB, one workgroup per CU; 256 workgroups at the prefill's 32,768 rows)
-// and has no barrier after they land.  Each wave owns 16 NB columns of a pass of 576 (NB <= 3)
+// these two shapes at 566 and 410 TFLOP/s).  Here a workgroup of 12 waves keeps its rows of
+// x (32 to 128, linear_launch) whole in LDS (128: 147 KB; one workgroup per CU; 256 of them at
+// the prefill's 32,768 rows) and has no barrier after they land.  Each wave owns 16 NB columns of a pass of 576 (NB <= 3)
 // and all rows: a weight fragment, loaded from L2 two k-steps ahead, feeds 8 MFMAs, so per
 // k-step a CU reads 36 KB of weights and 96 KB of LDS under 1,152 cycles of MFMAs per SIMD.
 //
@@ -163,24 +163,42 @@ __global__ void __launch_bounds__(LN_THREADS, 3) linear_kernel(LinearArgs a) {
 
 template <int DT>
 static int linear_launch(const LinearArgs& a, hipStream_t s) {
-  // The smallest row tile whose workgroups (one per CU) still fit one round of the chip, so
-  // that every CU has work and none has two tiles: 32, 64, else 128 rows.  A tile's columns
-  // are split over a workgroup per pass while those fit too.  Measured per call, N = 960 and
-  // N = 576 with the residual in place, against the library's GEMM (us):
-  //   rows   256: 9.0 / 9.1 (22 / 20)      4096: 11.0 / 10.2 (21 / 20)
-  //        10006: 19.3 / 14.2 (27 / 20)   16384: 24.9 / 19.7 (37 / 27)
-  //        20000: 34.1 / 29.3 (45 / 24)   32768: 41.1 / 34.9 (56 / 47)
-  // 10006 rows in 128-row tiles (79 workgroups a pass) took 25.2 and in 32-row tiles (313,
-  // two rounds) 22.5.
+  // One workgroup per CU.  32- and 64-row tiles while they fit one round of the chip; past that
+  // 80, 96, 112 or 128 rows, by the time of their rounds: a round of 16 mr rows takes about 4 (mr
+  // + 1/2) us at N = 576, so 17,000 rows are one round of 80-row tiles rather than one, half
+  // empty, of 128-row ones.  A tile's columns are split over a workgroup per pass while those
+  // fit too.  Measured per call, N = 960 and N = 576 with the residual in place, against the
+  // library's GEMM (us):
+  //   rows   256:   8.6 /   9.0 ( 21 /  18)     4096:  10.7 /   9.7 ( 21 /  18)
+  //        10006:  18.9 /  14.8 ( 27 /  18)    16384:  24.7 /  19.1 ( 37 /  27)
+  //        17000:  25.4 /  20.2 ( 45 /  22)    20000:  27.9 /  22.0 ( 46 /  24)
+  //        24000:  31.9 /  25.1 ( 43 /  41)    28000:  35.8 /  28.7 ( 65 /  48)
+  //        32768:  41.2 /  34.1 ( 57 /  46)    36000:  50.6 /  39.9 ( 62 /  54)
+  //        50000:  66.3 /  52.0 ( 81 /  64)    65536:  81.8 /  66.3 (110 /  65)
+  //        98304: 127.9 /  96.2 (149 / 110)   131072: 167.2 / 134.4 (200 / 127)
+  //       262144: 329.9 / 297.1 (391 / 256)
+  // (With 128-row tiles alone 17000 rows took 31.5 / 26.7, 36000 65.4 / 54.2.  From 60,000 rows
+  // on the library is up to 3 % faster at N = 576, from 131,072 more; every sublayer runs both,
+  // and the two together are faster here.)  The 128-row form spills 8 VGPRs; no other does.
   const int64_t cus = device_cus();
-  const int64_t t32 = cdiv(a.M, 32), t64 = cdiv(a.M, 64), t128 = cdiv(a.M, 128);
-  const int64_t tiles = t32 <= cus ? t32 : t64 <= cus ? t64 : t128;
-  const int64_t passes = cdiv(a.N, LN_PASS);
+  int mr = 2;
+  if (cdiv(a.M, 64) > cus) {
+    auto cost = [&](int r) { return cdiv(cdiv(a.M, 16 * r), cus) * (2 * r + 1); };
+    mr = 8;
+    for (int r = 7; r >= 5; --r)
+      if (cost(r) < cost(mr)) mr = r;
+  } else if (cdiv(a.M, 32) > cus) {
+    mr = 4;
+  }
+  const int64_t tiles = cdiv(a.M, 16 * mr), passes = cdiv(a.N, LN_PASS);
   NSMOE_REQUIRE(tiles < INT32_MAX, "linear: too many rows");
   const dim3 grid((unsigned)tiles, tiles * passes <= cus ? (unsigned)passes : 1u);
   KernelTimer timer("linear", s);
-  if (t32 <= cus) linear_kernel<DT, 2><<<grid, LN_THREADS, 0, s>>>(a);
-  else if (t64 <= cus) linear_kernel<DT, 4><<<grid, LN_THREADS, 0, s>>>(a);
+  if (mr == 2) linear_kernel<DT, 2><<<grid, LN_THREADS, 0, s>>>(a);
+  else if (mr == 4) linear_kernel<DT, 4><<<grid, LN_THREADS, 0, s>>>(a);
+  else if (mr == 5) linear_kernel<DT, 5><<<grid, LN_THREADS, 0, s>>>(a);
+  else if (mr == 6) linear_kernel<DT, 6><<<grid, LN_THREADS, 0, s>>>(a);
+  else if (mr == 7) linear_kernel<DT, 7><<<grid, LN_THREADS, 0, s>>>(a);
   else linear_kernel<DT, 8><<<grid, LN_THREADS, 0, s>>>(a);
   timer.stop();
   return check_launch("linear_kernel");

@@ -202,3 +202,19 @@ def test_captured_projections_share_kept_packs():
         torch.cuda.synchronize()
         assert torch.equal(out, ref) and len(spare) == 8 and gains_and_tables
     PACKS.clear()
+
+
+@pytest.mark.parametrize("M", [16385, 20480, 20481, 24577, 28673, 32769, 41000, 50000])
+def test_linear_row_tiles_of_long_calls(M):
+    """Row counts that choose tiles of 80, 96, 112 and 128 rows (256 CUs: one round, then two),
+    whole and ragged at the end, against the same rows in calls of at most 8,000 (32-row tiles):
+    a row's products are summed in the same order whatever its tile, so the bits are equal."""
+    x, w, r = _operands(M, 96, 592, torch.bfloat16, M)
+    wp = pack_linear(w)
+    print(f"[linear] {M} rows", flush=True)
+    for resid in (None, r):
+        got = linear(x, wp, 592, resid)
+        for s in range(0, M, 8000):
+            part = slice(s, min(M, s + 8000))
+            want = linear(x[part], wp, 592, None if resid is None else resid[part].contiguous())
+            assert torch.equal(got[part], want), s
