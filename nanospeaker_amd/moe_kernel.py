@@ -80,12 +80,25 @@ def _l_cap(m: int, n_experts: int) -> int:
     return -(-(m + min(n_experts, m) * (ALIGN_M - 1)) // ALIGN_M) * ALIGN_M
 
 
+def _private(module, name: str):
+    """A name of torch that it does not document, or None in a torch without it: what uses
+    it then takes the documented way."""
+    return getattr(module, name, None)
+
+
+_raw_stream = _private(torch._C, "_cuda_getCurrentRawStream")
+_interpreter_stack = _private(_private(torch._C, "_functorch"), "peek_interpreter_stack")
+_tracing_state = _private(torch._C, "_get_tracing_state")
+
+
 def _stream(device_index: "int | None" = None) -> int:
     """The handle of the current stream of a device (the current one by default), without
-    building the stream object (0.4 against 2.9 us a call)."""
+    building the stream object where torch allows it (0.4 against 2.9 us a call)."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device_index).cuda_stream
     if device_index is None:
         device_index = torch.cuda.current_device()
-    return torch._C._cuda_getCurrentRawStream(device_index)
+    return _raw_stream(device_index)
 
 
 def _p(t: Optional[Tensor]) -> Optional[int]:
@@ -1265,10 +1278,12 @@ def _block_fwd_infer(*inputs):
 def _plain_inference() -> bool:
     """Whether nothing can ask an eager call for a derivative or a transform: gradients off,
     no torch.func transform, no forward-mode level and no jit trace.  The autograd node
-    (which raises for the transforms it does not know) is then skipped."""
-    return (not torch.is_grad_enabled() and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0
-            and torch._C._get_tracing_state() is None)
+    (which raises for the transforms it does not know) is then skipped.  A torch that cannot
+    be asked keeps the node."""
+    return (not torch.is_grad_enabled()
+            and _interpreter_stack is not None and _interpreter_stack() is None
+            and getattr(torch.autograd.forward_ad, "_current_level", 0) < 0
+            and _tracing_state is not None and _tracing_state() is None)
 
 
 def block_forward(x, router_W, w_in, w_out, w_sh_in, w_sh_out, b_in, b_out, b_sh_in, b_sh_out,

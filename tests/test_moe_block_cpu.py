@@ -250,3 +250,27 @@ def test_the_autograd_node_is_skipped_only_for_plain_inference():
         assert mk._plain_inference()
     with torch.inference_mode():
         assert mk._plain_inference()
+
+
+def test_a_torch_without_the_undocumented_names_still_runs(monkeypatch):
+    """The stream handle and the questions behind _plain_inference use names that torch does
+    not document: without one of them the stream object is asked, and the node is kept."""
+    import types
+
+    from nanospeaker_amd import moe_kernel as mk
+
+    assert mk._private(None, "x") is None and mk._private(torch._C, "no_such_name") is None
+    with torch.no_grad():
+        for where, name in ((torch.autograd.forward_ad, "_current_level"),
+                            (mk, "_interpreter_stack"), (mk, "_tracing_state")):
+            assert mk._plain_inference()
+            with monkeypatch.context() as m:
+                if where is mk:
+                    m.setattr(where, name, None)
+                else:
+                    m.delattr(where, name)
+                assert not mk._plain_inference(), name
+    monkeypatch.setattr(mk, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda device=None: types.SimpleNamespace(cuda_stream=(7, device)))
+    assert mk._stream() == (7, None) and mk._stream(1) == (7, 1)
