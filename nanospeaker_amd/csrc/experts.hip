@@ -1017,6 +1017,15 @@ static int64_t tile_grid(const ExpParams& p, int bm) {  // upper bound on the ti
   return cdiv(M, bm) + std::min<int64_t>(M, p.E) + (int64_t)p.S * cdiv(p.T, bm);
 }
 
+// p for a launch of `grid` tiles of this file's kernels: runs of at most an eighth of them, so
+// that a small grid too keeps neighbouring tiles, which share a group's weights, on one XCD (d
+// 572, H 124, top-2 of 16 + 1, bf16: a forward of 1024 tokens, 64 tiles, took 90.4 us with its
+// tiles dealt singly and takes 85.7; 1531 tokens 93.4 and 89.0).
+static ExpParams with_run(ExpParams p, int64_t grid) {
+  p.xcd_run = (int)std::clamp<int64_t>(grid / 8, 1, p.xcd_run);
+  return p;
+}
+
 template <int DT>
 static int launch_fwd_tiles(const ExpParams& p, int nbw, int64_t grid, hipStream_t s) {
   if (grid <= 0) return NSMOE_OK;
@@ -1025,9 +1034,10 @@ static int launch_fwd_tiles(const ExpParams& p, int nbw, int64_t grid, hipStream
   KernelTimer timer("expert_fwd", s);
   constexpr int MR = gen_row_blocks(DT);
   const unsigned gr = (unsigned)tile_grid(p, 16 * MR);
-  if (nbw == 1) expert_fwd_kernel<DT, 1, MR><<<gr, NT, 0, s>>>(p);
-  else if (nbw == 2) expert_fwd_kernel<DT, 2, MR><<<gr, NT, 0, s>>>(p);
-  else if constexpr (DT != DT_F32) expert_fwd_kernel<DT, 4, MR><<<gr, NT, 0, s>>>(p);
+  const ExpParams q = with_run(p, gr);
+  if (nbw == 1) expert_fwd_kernel<DT, 1, MR><<<gr, NT, 0, s>>>(q);
+  else if (nbw == 2) expert_fwd_kernel<DT, 2, MR><<<gr, NT, 0, s>>>(q);
+  else if constexpr (DT != DT_F32) expert_fwd_kernel<DT, 4, MR><<<gr, NT, 0, s>>>(q);
   timer.stop();
   return check_launch("expert_fwd_kernel");
 }
@@ -1210,9 +1220,10 @@ static int experts_bwd_impl(const nsmoe_experts_args* a, const int32_t* inv, con
     KernelTimer timer("expert_bwd", s);
     constexpr int MR = gen_row_blocks(DT);
     const unsigned gr = (unsigned)tile_grid(p, 16 * MR);
-    if (nbw == 1) expert_bwd_kernel<DT, 1, MR><<<gr, NT, 0, s>>>(p);
-    else if (nbw == 2) expert_bwd_kernel<DT, 2, MR><<<gr, NT, 0, s>>>(p);
-    else if constexpr (DT != DT_F32) expert_bwd_kernel<DT, 4, MR><<<gr, NT, 0, s>>>(p);
+    const ExpParams q = with_run(p, gr);
+    if (nbw == 1) expert_bwd_kernel<DT, 1, MR><<<gr, NT, 0, s>>>(q);
+    else if (nbw == 2) expert_bwd_kernel<DT, 2, MR><<<gr, NT, 0, s>>>(q);
+    else if constexpr (DT != DT_F32) expert_bwd_kernel<DT, 4, MR><<<gr, NT, 0, s>>>(q);
     timer.stop();
     NSMOE_TRY(check_launch("expert_bwd_kernel"));
   }
