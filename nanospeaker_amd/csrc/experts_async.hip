@@ -10,8 +10,8 @@
 // copies and frees the ring slot the next issue overwrites.
 //
 // Taken for bf16 / fp16 when d and H are multiples of 8, the operands are 16-byte aligned
-// and H <= 128 (the ring and the h tile fit one workgroup's LDS); other shapes use the
-// register-staged kernels.
+// and H <= 128 (the ring and the h tile fit one workgroup's LDS); dW also for fp32 and any
+// H.  Other shapes use the register-staged kernels.
 #include <stdlib.h>
 
 #include <algorithm>
@@ -1699,7 +1699,8 @@ static void dx_reg_launch(const ExpParams& p, int mb, int dist, hipStream_t s) {
     // workgroup per pass instead of one for all of them divides a tile's chain of k-steps
     // by three and copies nothing twice (this kernel copies its rows for every pass anyway).
     // expert_dx 20.4 -> 11.4 us at T = 150, 22.3 -> 16.0 at 1024, 26.9 -> 21.7 at 2047, 33.8
-    // -> 32.0 at 4096, 42.2 -> 42.5 at 6000.  The k loop unrolls by the prefetch distance.
+    // -> 32.0 at 4096 (the last that takes them; at 6000, forced, 42.2 -> 42.5).  The k loop
+    // unrolls by the prefetch distance: other step counts keep one workgroup a tile.
     ExpParams q = p;
     const int npass = (p.d + NP2 - 1) / NP2, nkk = 2 * p.H / 32;
     q.dx_split = nkk % dist == 0 ? npass : 1;

@@ -111,6 +111,19 @@ def assert_close_bf16(name, got, ref, max_abs=BF16_MAX_ABS, rel_l2=BF16_REL_L2):
                 f"rel-L2 {rl2:.3e} (<= {rel_l2})")
 
 
+def dw_rows_per_chunk(d, H, T, k, S):
+    """The row chunks of the dW work: at least 36, and more where few output tiles (192 x 128
+    and 128 x 192 on the ring kernel, 64 x 128 and 128 x 64 off the vector path) would leave
+    the launch short of items; 512 to 8192 rows each, whole 32s."""
+    up = lambda a, b: -(-a // b)
+    if d % 8 == 0 and H % 8 == 0:
+        tiles, items = up(d, 192) * up(2 * H, 128) + up(H, 128) * up(d, 192), 324
+    else:
+        tiles, items = up(d, 64) * up(2 * H, 128) + up(H, 128) * up(d, 64), 1152
+    rc = up(T * (k + S), max(36, up(items, tiles)) * 32) * 32
+    return min(max(rc, 512), 8192)
+
+
 @contextmanager
 def lib_options(**values):
     """Sets libnsmoe tuning options (nsmoe_set_option) for the body, then restores 0."""

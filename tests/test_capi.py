@@ -13,6 +13,7 @@ import pytest
 
 from nanospeaker_amd import _native as nat
 from nanospeaker_amd import moe_kernel as mk
+from tests.helpers import dw_rows_per_chunk
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "nsmoe.h"
 
@@ -129,19 +130,6 @@ def test_workspace_sizes_are_positive_and_grow():
     # [chunks, E] int32 histograms; chunks of 1024 pairs while E <= 256, else 256
     assert nat.lib().nsmoe_dispatch_workspace_size(49152, 76) == 48 * 76 * 4
     assert nat.lib().nsmoe_dispatch_workspace_size(49152, 1000) == 192 * 1000 * 4
-
-
-def dw_rows_per_chunk(d, H, T, k, S):
-    """The row chunks of the dW work: at least 36, and more where few output tiles (192 x 128
-    and 128 x 192 on the ring kernel, 64 x 128 and 128 x 64 off the vector path) would leave
-    the launch short of items; 512 to 8192 rows each, whole 32s."""
-    up = lambda a, b: -(-a // b)
-    if d % 8 == 0 and H % 8 == 0:
-        tiles, items = up(d, 192) * up(2 * H, 128) + up(H, 128) * up(d, 192), 324
-    else:
-        tiles, items = up(d, 64) * up(2 * H, 128) + up(H, 128) * up(d, 64), 1152
-    rc = up(T * (k + S), max(36, up(items, tiles)) * 32) * 32
-    return min(max(rc, 512), 8192)
 
 
 @pytest.mark.parametrize("d,H,E,k,S,T", [

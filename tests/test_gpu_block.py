@@ -30,7 +30,7 @@ import pytest
 import torch
 
 from oracle import moe_ref as R
-from tests.helpers import assert_close_bf16
+from tests.helpers import assert_close_bf16, dw_rows_per_chunk
 
 pytestmark = pytest.mark.gpu
 
@@ -217,13 +217,14 @@ def test_skewed_T16384_forward_backward_block_path():
 
 
 def test_skewed_T8192_forward_backward_block_path():
-    """The headline shape under the Zipf offset: T k = 49,152 pairs sit below E x 691, so
-    the dW split-K reduce inside combine_dx's launch takes the routed groups in its one
-    looping row, and with ~15 % of the pairs on the hot expert several routed groups span
-    more than one 768-row chunk and are reduced there one after another."""
+    """The headline shape under the Zipf offset: with ~15 % of the pairs on the hot expert
+    several routed groups span more than one dW chunk (1824 rows), so that with the two
+    shared ones the split-K reduce inside combine_dx's launch has more items (216 a group)
+    than its 864 workgroups."""
     bias = torch.from_numpy(np.load(ZIPF, allow_pickle=False)).float()
     ref = run_case(8192, train=True, backward=True, logit_bias=bias)
-    assert int((ref.counts > 768).sum()) >= 2
+    rc = dw_rows_per_chunk(576, 128, 8192, 6, 2)
+    assert rc == 1824 and int((ref.counts > rc).sum()) > 2
 
 
 def test_prefill_layer_T32768_eval():
@@ -284,12 +285,14 @@ def test_dw_ring_stages(stages, T):
 
 @pytest.mark.parametrize("T", [15, 63, 65, 400])
 @pytest.mark.parametrize("cfg", [dict(), dict(d=320, E=12, k=3, S=1, d_ff=192),
-                                 dict(d=384, E=10, k=2, S=0, d_ff=144), dict(d=128, E=6, k=2, S=2,
-                                                                             d_ff=96)])
+                                 dict(d=384, E=10, k=2, S=0, d_ff=144),
+                                 dict(d=384, E=10, k=2, S=1, d_ff=72),
+                                 dict(d=128, E=6, k=2, S=2, d_ff=96)])
 def test_dx_passes_split_over_workgroups(T, cfg):
     """Small calls give every pass of 192 dX columns a workgroup of its own: three passes, two
-    with a ragged second one (d 320), an odd number of k-steps (H 96, two of three 64-row
-    steps: not split) and a single pass, at the edges of a 64-row tile.  (Not at T = 1: with
+    with a ragged second one (d 320), two whole ones (d 384), two that share a workgroup
+    because their three k-steps (H 48) are no multiple of the prefetch distance, and a single
+    pass, at the edges of a 64-row tile.  (Not at T = 1: with
     two experts a token the router's gradient there is one difference of two gate gradients
     rounded to bf16, 2^-9 of each, whose relative error has no bound of 5e-3.)"""
     run_case(T, train=True, backward=True, **cfg)

@@ -72,3 +72,24 @@ def test_dw_pair_kernel_fits_twice_in_a_cu(kernels):
     for pattern, rows in ((r"dw_pair_kernelILi[012]ELi2E", 8192), (r"dw_pair_kernelILi[01]ELi3E", 5000)):
         for name, k in _of(kernels, pattern).items():
             assert 2 * (k["lds"] + 4 * rows) <= LDS_PER_CU, (name, k)
+
+
+@pytest.mark.parametrize("pattern,spills", [
+    (r"expert_fwd_reg_kernelILi0ELi2ELi6ELi2ELb0E", 3),      # 96-row tiles
+    (r"expert_fwd_reg_kernelILi0ELi2ELi[24]ELi[26]ELb[01]E", 0),
+    (r"expert_bwd_reg_kernelILi0ELi2ELi2ELi[36]ELb[01]E", 0),
+    (r"expert_bwd_reg_kernelILi0ELi2ELi3ELi4ELb1E", 0),
+    (r"expert_dx_reg_kernelILi0ELi2ELi4E", 0),
+    (r"expert_dx_res_kernelILi0ELi2E", 0),
+    (r"dw_pair_kernelILi[012]ELi2E", 0),
+    (r"dw_kernelILi[012]E", 0),
+    (r"expert_fwd_kernelILi[012]E", 0),
+    (r"expert_bwd_kernelILi[01]E", 0),
+    (r"expert_bwd_kernelILi2E", 6),                          # fp32
+    (r"linear_kernelILi[01]ELi[24567]E", 0),
+    (r"linear_kernelILi[01]ELi8E", 8),                       # 128 rows
+    (r"attn_fwd_kernel", 0), (r"router_fwd_kernel", 0), (r"combine_dx_kernel", 0)])
+def test_registers_spilled_by_the_kernels_taken_by_default(kernels, pattern, spills):
+    """The forms that the launch rules take without an option: what each keeps in scratch."""
+    for name, k in _of(kernels, pattern).items():
+        assert k["spills"] <= spills, (name, k)
