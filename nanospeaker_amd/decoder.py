@@ -163,11 +163,11 @@ def _fragments(w: torch.Tensor) -> torch.Tensor:
     return w.reshape(k // 32, 4, 8, n // 16, 16).permute(3, 0, 1, 4, 2)
 
 
-@torch.inference_mode()  # refresh() also writes buffers that were made in inference mode
 def _pack_projection(weights, into: torch.Tensor) -> None:
     """The weights side by side, cast and written in place: in nsmoe_linear's order, or as the
     plain matrix where `into` has its two dimensions."""
-    w = (torch.cat(tuple(weights), dim=1) if len(weights) > 1 else weights[0]).to(into.dtype)
+    w = torch.cat(tuple(weights), dim=1) if len(weights) > 1 else weights[0]
+    w = w.detach().to(into.dtype)
     into.copy_(w if into.dim() == 2 else _fragments(w))
 
 

@@ -488,7 +488,8 @@ class PackCache:
                 if any(k is None for k in keys) or entry.spec is None:
                     continue
                 if callable(entry.spec):
-                    entry.spec(keys, entry.p_in)
+                    with torch.inference_mode():  # the buffer may have been made in it
+                        entry.spec(keys, entry.p_in)
                 else:
                     _pack_experts(entry.spec, keys, entry.p_in, entry.p_out)
                 entry.states = tuple(self._state(k) for k in keys)

@@ -1,8 +1,9 @@
 """
 nsmoe_linear (nanospeaker_amd/csrc/linear.hip) against the same product in 64 bits: x W and
-x W + resid with one rounding of the fp32 sum, at the edges of its row tiles (32, 64 and 128 rows) and of the row counts that choose them,
-of a wave's 48, 32 and 16 columns and of a pass of 576, and through the attention sublayer
-with operands the kernel cannot read in place.
+x W + resid with one rounding of the fp32 sum, at the edges of its row tiles (32 to 128 rows)
+and of the row counts that choose them, of a wave's 48, 32 and 16 columns and of a pass of 576,
+and through the attention sublayer with operands the kernel cannot read in place; and the
+packed weights it reads, across streams, captures and updates.
 """
 
 import pytest
