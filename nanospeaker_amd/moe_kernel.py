@@ -281,7 +281,9 @@ class _PackEntry:
     def valid_for(self, keys) -> bool:
         """Whether `keys` are the tensors this was packed from, unchanged."""
         for ref, state, k in zip(self.refs, self.states, keys):
-            if ref() is not k or state != PackCache._state(k):
+            # PackCache._state(k), without the call: this runs for every kernel call
+            if ref() is not k or state != (k.data_ptr(), k.shape, k.stride(), k.dtype,
+                                           k._version):
                 return False
         return True
 
